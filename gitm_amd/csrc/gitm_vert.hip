@@ -2,12 +2,19 @@
 // the single-grid step, the column prep, errors and the host-array entry.
 //
 // Entry points are declared in include/gitm_vert.h.  One workgroup per
-// column (the column of workgroup blockIdx.x is xcd_column's), NT = 64*W threads,
-// one level per thread; see vert_column.h for the column algorithm.
+// column (the column of workgroup blockIdx.x is xcd_column's): the AUSM step
+// with NG lanes per level (gitm_vert_ausm.hip), the Rusanov step with NT = 64*W
+// threads, one level per thread (vert_column.h).
 #include "vert_gpu.h"
+#include "vert_group.h"
+
+// gitm_vert_ausm.hip
+void launch_ausm(unsigned ncols, hipStream_t stream, const gv::KParams &kp,
+                 const gitm_vert_columns &c);
 
 namespace {
 
+// The Rusanov step, one lane per level (vert_column.h).
 template <int NT, int SOLVER, bool IONS>
 __global__ void __launch_bounds__(NT) vert_column_kernel(gv::KParams kp, gitm_vert_columns io) {
   extern __shared__ double lds[];
@@ -17,26 +24,34 @@ __global__ void __launch_bounds__(NT) vert_column_kernel(gv::KParams kp, gitm_ve
 }
 
 // One thread per level: blockDim = nAlts+4 (<= NT, the compile-time bound).
-template <int NT, bool IONS>
-void launch_ions(int solver, dim3 grid, hipStream_t stream, const gv::KParams &kp,
-                 const gitm_vert_columns &c) {
+template <int NT>
+void launch_rusanov(dim3 grid, hipStream_t stream, const gv::KParams &kp,
+                    const gitm_vert_columns &c) {
   const dim3 block(kp.n_alts + 4);
-  const size_t lds = gv::lds_bytes(kp.n_alts, IONS, gv::carry_in_lds(NT / 64));
-  if (solver == GITM_VERT_AUSM)
-    hipLaunchKernelGGL((vert_column_kernel<NT, GITM_VERT_AUSM, IONS>), grid, block, lds,
+  const size_t lds = gv::lds_bytes(kp.n_alts, kp.ions != 0, gv::carry_in_lds(NT / 64));
+  if (kp.ions)
+    hipLaunchKernelGGL((vert_column_kernel<NT, GITM_VERT_RUSANOV, true>), grid, block, lds,
                        stream, kp, c);
   else
-    hipLaunchKernelGGL((vert_column_kernel<NT, GITM_VERT_RUSANOV, IONS>), grid, block, lds,
+    hipLaunchKernelGGL((vert_column_kernel<NT, GITM_VERT_RUSANOV, false>), grid, block, lds,
                        stream, kp, c);
 }
 
-template <int NT>
-void launch(int solver, dim3 grid, hipStream_t stream, const gv::KParams &kp,
-            const gitm_vert_columns &c) {
-  if (kp.ions)
-    launch_ions<NT, true>(solver, grid, stream, kp, c);
-  else
-    launch_ions<NT, false>(solver, grid, stream, kp, c);
+int launch(int solver, int waves, unsigned ncols, hipStream_t stream, const gv::KParams &kp,
+           const gitm_vert_columns &c) {
+  if (solver == GITM_VERT_AUSM) {
+    launch_ausm(ncols, stream, kp, c);
+    return GITM_VERT_OK;
+  }
+  const dim3 grid(ncols);
+  switch (waves) {
+    case 1: launch_rusanov<64>(grid, stream, kp, c); break;
+    case 2: launch_rusanov<128>(grid, stream, kp, c); break;
+    case 3: launch_rusanov<192>(grid, stream, kp, c); break;
+    case 4: launch_rusanov<256>(grid, stream, kp, c); break;
+    default: return GITM_VERT_EINVAL;
+  }
+  return GITM_VERT_OK;
 }
 
 template <int NT>
@@ -134,7 +149,11 @@ int gitm_vert_advance(gitm_vert_handle *h, const gitm_vert_params *p,
   if (!gv::valid_waves(waves) || !gv::tile_fits(waves, c->n_alts)) return GITM_VERT_EINVAL;
   GV_HIP(hipSetDevice(h->device));
   gv::KParams kp = gv::make_kparams(p, c, solver, n_steps, h->d_err);
-  kp.scr_fields = gv::scratch_fields(gv::carry_in_lds(waves), kp.ions != 0);
+  // carries in device memory: of the kernels with one lane per level (which the
+  // AUSM step uses only for columns with ions that vert_group.h does not fit)
+  kp.scr_fields = solver == GITM_VERT_AUSM && gv::group_fits(c->n_alts, kp.ions != 0)
+                      ? 0
+                      : gv::scratch_fields(gv::carry_in_lds(waves), kp.ions != 0);
   const size_t need = (size_t)ncols * kp.scr_fields * (size_t)(c->n_alts + 4) * sizeof(double);
   if (h->scratch_bytes < need) {
     if (h->scratch) {
@@ -148,14 +167,8 @@ int gitm_vert_advance(gitm_vert_handle *h, const gitm_vert_params *p,
     h->scratch_bytes = need;
   }
   kp.scratch = h->scratch;
-  const dim3 grid(ncols);
-  switch (waves) {
-    case 1: launch<64>(solver, grid, h->stream, kp, *c); break;
-    case 2: launch<128>(solver, grid, h->stream, kp, *c); break;
-    case 3: launch<192>(solver, grid, h->stream, kp, *c); break;
-    case 4: launch<256>(solver, grid, h->stream, kp, *c); break;
-    default: return GITM_VERT_EINVAL;
-  }
+  rc = launch(solver, waves, (unsigned)ncols, h->stream, kp, *c);
+  if (rc) return rc;
   GV_HIP(hipGetLastError());
   return GITM_VERT_OK;
 }
@@ -388,14 +401,8 @@ extern "C" int gitm_vert_advance_noalloc(const gitm_vert_params *p, const gitm_v
   gv::KParams kp = gv::make_kparams(p, c, solver, n_steps, err);
   kp.scr_fields = fields;
   kp.scratch = base + kNoallocCarryOffset;
-  const dim3 grid((unsigned)ncols);
-  switch (waves) {
-    case 1: launch<64>(solver, grid, stream, kp, *c); break;
-    case 2: launch<128>(solver, grid, stream, kp, *c); break;
-    case 3: launch<192>(solver, grid, stream, kp, *c); break;
-    case 4: launch<256>(solver, grid, stream, kp, *c); break;
-    default: return GITM_VERT_EINVAL;
-  }
+  rc = launch(solver, waves, (unsigned)ncols, stream, kp, *c);
+  if (rc) return rc;
   if (err_word) hipLaunchKernelGGL(copy_word, dim3(1), dim3(1), 0, stream, err_word, err);
   GV_HIP(hipGetLastError());
   return GITM_VERT_OK;

@@ -1,0 +1,86 @@
+// gitm_vert_ausm.hip -- the AUSM step of a single grid and of a batch: one
+// workgroup per column, NG lanes per level (vert_group.h).
+#include "vert_gpu.h"
+#include "vert_group.h"
+
+namespace {
+
+// 768 threads hold the tallest column; three wavefronts per SIMD leave a lane
+// 168 registers.
+template <bool IONS>
+__global__ void __launch_bounds__(768, 4)
+    vert_group_kernel(gv::KParams kp, gitm_vert_columns io) {
+  extern __shared__ double lds[];
+  GpuCtx cx{kp.err};
+  const int col = xcd_column((int)blockIdx.x, (int)gridDim.x);
+  gv::run_group_column<IONS>(cx, kp, io, col, lds, kp.dt, col, kp.n_alts);
+}
+
+// One workgroup per column of the members mem[0..n-1], whose first_block
+// numbers the launch's columns; workgroups are as wide as the widest of them
+// needs.
+template <bool IONS>
+__global__ void __launch_bounds__(768, 4)
+    vert_group_batch_kernel(gv::KParams kp, const BatchMember *__restrict__ mem, int n,
+                            const double *__restrict__ dt_dev) {
+  extern __shared__ double lds[];
+  GpuCtx cx{kp.err};
+  const int b = xcd_column((int)blockIdx.x, (int)gridDim.x);
+  const BatchMember &e = mem[find_member(mem, n, b)];
+  if ((int)threadIdx.x >= gv::group_threads(e.io.n_alts)) return;
+  const int col = b - e.first_block;
+  gv::run_group_column<IONS>(cx, kp, e.io, col, lds, dt_dev ? dt_dev[e.member] : kp.dt,
+                             e.col_offset + col, e.io.n_alts);
+}
+
+// Columns with ions too tall for vert_group_kernel's LDS: one lane per level
+// (vert_column.h), the RK4 carries in device memory.
+__global__ void __launch_bounds__(256)
+    vert_tall_ion_kernel(gv::KParams kp, gitm_vert_columns io, double *scratch,
+                         const double *dt_dev, int err_first) {
+  extern __shared__ double lds[];
+  GpuCtx cx{kp.err};
+  const int col = xcd_column((int)blockIdx.x, (int)gridDim.x);
+  gv::run_column<256, GITM_VERT_AUSM, true, false>(cx, kp, io, col, lds, scratch,
+                                                   dt_dev ? *dt_dev : kp.dt, err_first + col,
+                                                   io.n_alts, gv::scratch_fields(false, true));
+}
+
+}  // namespace
+
+// Queues the step of one grid's (or one batch member's) columns with ions that
+// group_fits refuses; scratch: scratch_fields(false, true) doubles per level.
+void launch_ausm_tall_ions(unsigned ncols, hipStream_t stream, const gv::KParams &kp,
+                           const gitm_vert_columns &c, double *scratch, const double *dt_dev,
+                           int err_first) {
+  hipLaunchKernelGGL(vert_tall_ion_kernel, dim3(ncols), dim3(c.n_alts + 4),
+                     gv::lds_bytes(c.n_alts, true, false), stream, kp, c, scratch, dt_dev,
+                     err_first);
+}
+
+// Queues the step of `ncols` columns of the n members at mem, none taller than
+// n_alts.
+void launch_ausm_batch(unsigned ncols, int n_alts, hipStream_t stream, const gv::KParams &kp,
+                       const BatchMember *mem, int n, const double *dt_dev) {
+  const dim3 grid(ncols), block(gv::group_threads(n_alts));
+  const size_t lds = gv::group_lds_bytes(n_alts, kp.ions != 0);
+  if (kp.ions)
+    hipLaunchKernelGGL(vert_group_batch_kernel<true>, grid, block, lds, stream, kp, mem, n,
+                       dt_dev);
+  else
+    hipLaunchKernelGGL(vert_group_batch_kernel<false>, grid, block, lds, stream, kp, mem, n,
+                       dt_dev);
+}
+
+// One column per workgroup of c's ncols columns.
+void launch_ausm(unsigned ncols, hipStream_t stream, const gv::KParams &kp,
+                 const gitm_vert_columns &c) {
+  const dim3 grid(ncols), block(gv::group_threads(kp.n_alts));
+  const size_t lds = gv::group_lds_bytes(kp.n_alts, kp.ions != 0);
+  if (!gv::group_fits(kp.n_alts, kp.ions != 0))
+    launch_ausm_tall_ions(ncols, stream, kp, c, kp.scratch, nullptr, 0);
+  else if (kp.ions)
+    hipLaunchKernelGGL(vert_group_kernel<true>, grid, block, lds, stream, kp, c);
+  else
+    hipLaunchKernelGGL(vert_group_kernel<false>, grid, block, lds, stream, kp, c);
+}

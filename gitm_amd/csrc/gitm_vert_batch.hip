@@ -1,15 +1,24 @@
 // gitm_vert_batch.hip -- ensemble batches of the vertical step (the
 // gitm_vert_batch_* entry points of include/gitm_vert.h).
 //
-// A batch step is one launch of vert_ensemble_kernel (gitm_vert_ensemble.hip,
-// one object per workgroup size) over a task list: the columns of more than
-// 64 levels one workgroup each, then the shorter columns one wavefront each,
-// several per workgroup.  The batch prep is one launch as well.
+// The AUSM step of a batch is one launch per class of column heights
+// (gitm_vert_ausm.hip).  A Rusanov step is one launch of vert_ensemble_kernel
+// (gitm_vert_ensemble.hip, one object per workgroup size) over a task list: the
+// columns of more than 64 levels one workgroup each, then the shorter columns
+// one wavefront each, several per workgroup.  The batch prep is one launch.
 #include "vert_gpu.h"
+#include "vert_group.h"
+
+// gitm_vert_ausm.hip
+void launch_ausm_batch(unsigned ncols, int n_alts, hipStream_t stream, const gv::KParams &kp,
+                       const BatchMember *mem, int n, const double *dt_dev);
+void launch_ausm_tall_ions(unsigned ncols, hipStream_t stream, const gv::KParams &kp,
+                           const gitm_vert_columns &c, double *scratch, const double *dt_dev,
+                           int err_first);
 
 #define GV_ENS_DECL(W)                                                                     \
-  int ensemble_occupancy_w##W(int solver, bool ions, size_t lds_bytes);                    \
-  hipError_t launch_ensemble_w##W(int solver, bool ions, int grid, size_t lds_bytes,       \
+  int ensemble_occupancy_w##W(bool ions, size_t lds_bytes);                                \
+  hipError_t launch_ensemble_w##W(bool ions, int grid, size_t lds_bytes,                   \
                                   hipStream_t stream, const gv::KParams &kp,               \
                                   const BatchMember *mem, const EnsLayout &lay,            \
                                   const double *dt_dev);
@@ -21,24 +30,24 @@ GV_ENS_DECL(4)
 
 namespace {
 
-int ensemble_occupancy(int waves, int solver, bool ions, size_t lds) {
+int ensemble_occupancy(int waves, bool ions, size_t lds) {
   switch (waves) {
-    case 1: return ensemble_occupancy_w1(solver, ions, lds);
-    case 2: return ensemble_occupancy_w2(solver, ions, lds);
-    case 3: return ensemble_occupancy_w3(solver, ions, lds);
-    case 4: return ensemble_occupancy_w4(solver, ions, lds);
+    case 1: return ensemble_occupancy_w1(ions, lds);
+    case 2: return ensemble_occupancy_w2(ions, lds);
+    case 3: return ensemble_occupancy_w3(ions, lds);
+    case 4: return ensemble_occupancy_w4(ions, lds);
     default: return 0;
   }
 }
 
-hipError_t launch_ensemble(int waves, int solver, bool ions, int grid, size_t lds,
+hipError_t launch_ensemble(int waves, bool ions, int grid, size_t lds,
                            hipStream_t stream, const gv::KParams &kp, const BatchMember *mem,
                            const EnsLayout &lay, const double *dt_dev) {
   switch (waves) {
-    case 1: return launch_ensemble_w1(solver, ions, grid, lds, stream, kp, mem, lay, dt_dev);
-    case 2: return launch_ensemble_w2(solver, ions, grid, lds, stream, kp, mem, lay, dt_dev);
-    case 3: return launch_ensemble_w3(solver, ions, grid, lds, stream, kp, mem, lay, dt_dev);
-    case 4: return launch_ensemble_w4(solver, ions, grid, lds, stream, kp, mem, lay, dt_dev);
+    case 1: return launch_ensemble_w1(ions, grid, lds, stream, kp, mem, lay, dt_dev);
+    case 2: return launch_ensemble_w2(ions, grid, lds, stream, kp, mem, lay, dt_dev);
+    case 3: return launch_ensemble_w3(ions, grid, lds, stream, kp, mem, lay, dt_dev);
+    case 4: return launch_ensemble_w4(ions, grid, lds, stream, kp, mem, lay, dt_dev);
     default: return hipErrorInvalidValue;
   }
 }
@@ -77,11 +86,19 @@ struct gitm_vert_batch {
   bool uniform_tall = true;  // every tall column needs the same wavefront count
   int tall_waves = 0;        // ... which is this one
   gitm_vert_batch_tile tile{};
-  int occupancy[2][2] = {};  // workgroups per CU of the tile's kernel [ausm][ions]
+  int occupancy[2] = {};  // workgroups per CU of the tile's kernel [ions]
   int slot[2] = {};          // short columns' LDS slot in doubles [ions]
   size_t lds[2] = {};        // LDS of a workgroup [ions]
   int n_cu = 0;
   size_t lds_max = 0;
+  // the AUSM step's launches: members by falling height, in classes whose
+  // columns fit a CU in the same number
+  struct Class {
+    int first, n, n_alts;  // members of the sorted table, the tallest's nAlts
+    long long cols;
+  };
+  std::vector<Class> classes[2];  // [ions]
+  BatchMember *d_sorted[2] = {};  // first_block counts within the class
   BatchMember *d_table = nullptr;
   double *scratch = nullptr;
   size_t scratch_bytes = 0;
@@ -94,6 +111,45 @@ long long member_columns(const gitm_vert_columns &c) {
 }
 
 int waves_of(int n_alts) { return (n_alts + 4 + 63) / 64; }
+
+// Columns of n_alts levels that a CU holds in the AUSM step: by its LDS, and by
+// its sixteen wavefronts, of which a workgroup takes a multiple of four.
+int ausm_columns_per_cu(int n_alts, bool ions, size_t lds_max) {
+  const int wf = (gv::NG * waves_of(n_alts) + 3) / 4 * 4;
+  return std::min<int>((int)(lds_max / (gv::group_lds_bytes(n_alts, ions) + 256)), 16 / wf);
+}
+
+// The AUSM step's classes.  A launch gives every workgroup the LDS and the
+// threads of its tallest column, and ends with a tail in which the chip
+// empties; so members are launched apart where shorter columns fit a CU in
+// greater number, and together where they are too few to fill it twice.
+int ausm_classes(gitm_vert_batch *b, bool ions) {
+  std::vector<BatchMember> m;
+  for (const BatchMember &e : b->table)
+    if (gv::group_fits(e.io.n_alts, ions)) m.push_back(e);
+  std::stable_sort(m.begin(), m.end(), [](const BatchMember &p, const BatchMember &q) {
+    return p.io.n_alts > q.io.n_alts;
+  });
+  std::vector<gitm_vert_batch::Class> &cl = b->classes[ions];
+  for (int i = 0; i < (int)m.size(); i++) {
+    const int na = m[i].io.n_alts;
+    if (cl.empty() || (ausm_columns_per_cu(na, ions, b->lds_max) !=
+                           ausm_columns_per_cu(cl.back().n_alts, ions, b->lds_max) &&
+                       cl.back().cols >= 2LL * b->n_cu *
+                                             ausm_columns_per_cu(cl.back().n_alts, ions,
+                                                                 b->lds_max)))
+      cl.push_back({i, 0, na, 0});
+    m[i].first_block = (int)cl.back().cols;
+    cl.back().n++;
+    cl.back().cols += (long long)m[i].io.n_lons * m[i].io.n_lats * m[i].io.n_blocks;
+  }
+  if (m.empty()) return GITM_VERT_OK;
+  if (hipMalloc(&b->d_sorted[ions], m.size() * sizeof(BatchMember)) != hipSuccess)
+    return GITM_VERT_ENOMEM;
+  GV_HIP(hipMemcpy(b->d_sorted[ions], m.data(), m.size() * sizeof(BatchMember),
+                   hipMemcpyHostToDevice));
+  return GITM_VERT_OK;
+}
 
 // LDS doubles of a short column of n_alts levels, rounded up to even so
 // that every slot starts 16-byte aligned
@@ -112,7 +168,7 @@ std::vector<int> place_carries(const gitm_vert_batch *b, const gitm_vert_batch_t
   std::vector<int> flag(b->table.size(), t.carries_in_lds ? 1 : 0);
   if (t.carries_in_lds != 2) return flag;
   const bool ions = b->ions != 0;
-  const int occ = std::max(1, ensemble_occupancy(t.waves_per_workgroup, GITM_VERT_AUSM, ions, 0));
+  const int occ = std::max(1, ensemble_occupancy(t.waves_per_workgroup, ions, 0));
   const size_t budget = b->lds_max / (size_t)occ;
   for (size_t i = 0; i < b->table.size(); i++) {
     const int na = b->table[i].io.n_alts;
@@ -203,12 +259,9 @@ int batch_layout(gitm_vert_batch *b) {
   for (int i = 0; i < 2; i++) {
     b->slot[i] = slot_doubles(b, i != 0, flag);
     b->lds[i] = tile_lds(b, b->tile, i != 0);
-    for (int s = 0; s < 2; s++)
-      b->occupancy[s][i] =
-          (i && !b->ions) ? 0
-                          : ensemble_occupancy(b->tile.waves_per_workgroup,
-                                               s ? GITM_VERT_AUSM : GITM_VERT_RUSANOV, i != 0,
-                                               b->lds[i]);
+    b->occupancy[i] = (i && !b->ions)
+                          ? 0
+                          : ensemble_occupancy(b->tile.waves_per_workgroup, i != 0, b->lds[i]);
   }
   return GITM_VERT_OK;
 }
@@ -283,6 +336,8 @@ int gitm_vert_batch_create(gitm_vert_handle *h, const gitm_vert_columns *members
     b->lds_max = (size_t)lds_max;
     b->tile = auto_tile(b);
     rc = check_tile(b, b->tile);
+    if (!rc) rc = ausm_classes(b, false);
+    if (!rc && b->ions) rc = ausm_classes(b, true);
     if (!rc) rc = batch_layout(b);
   }
   if (rc) {
@@ -298,6 +353,8 @@ int gitm_vert_batch_destroy(gitm_vert_batch *b) {
   (void)hipSetDevice(b->h->device);
   (void)hipStreamSynchronize(b->h->stream);
   if (b->d_table) (void)hipFree(b->d_table);
+  for (BatchMember *s : b->d_sorted)
+    if (s) (void)hipFree(s);
   if (b->scratch) (void)hipFree(b->scratch);
   delete b;
   return GITM_VERT_OK;
@@ -333,17 +390,33 @@ int gitm_vert_batch_advance(gitm_vert_batch *b, const gitm_vert_params *p, int s
   // nAlts and the carries' stride come from each member in the kernel
   gv::KParams kp = gv::make_kparams(p, &b->members[0], solver, n_steps, h->d_err);
   const bool ions = kp.ions != 0;
+  if (solver == GITM_VERT_AUSM) {
+    for (const gitm_vert_batch::Class &c : b->classes[ions]) {
+      launch_ausm_batch((unsigned)c.cols, c.n_alts, h->stream, kp, b->d_sorted[ions] + c.first,
+                        c.n, dt_device);
+      GV_HIP(hipGetLastError());
+    }
+    for (const BatchMember &e : b->table) {
+      if (gv::group_fits(e.io.n_alts, ions)) continue;
+      // (their carries are in the batch's scratch under every tile that fits)
+      launch_ausm_tall_ions((unsigned)member_columns(e.io), h->stream, kp, e.io,
+                            b->scratch + reinterpret_cast<size_t>(e.scratch),
+                            dt_device ? dt_device + e.member : nullptr, e.col_offset);
+      GV_HIP(hipGetLastError());
+    }
+    return GITM_VERT_OK;
+  }
   EnsLayout lay = b->lay;
   lay.slot_doubles = b->slot[ions];
   const size_t lds = b->lds[ions];
   int grid = lay.n_tasks;
   if (b->tile.persistent) {
-    const int occ = b->occupancy[solver == GITM_VERT_AUSM][ions];
+    const int occ = b->occupancy[ions];
     if (occ < 1) return GITM_VERT_EHIP;
     grid = std::min(grid, occ * b->n_cu);
   }
   if (grid < 1) return GITM_VERT_OK;
-  GV_HIP(launch_ensemble(b->tile.waves_per_workgroup, solver, ions, grid, lds, h->stream, kp,
+  GV_HIP(launch_ensemble(b->tile.waves_per_workgroup, ions, grid, lds, h->stream, kp,
                          b->d_table, lay, dt_device));
   GV_HIP(hipGetLastError());
   return GITM_VERT_OK;

@@ -1,4 +1,5 @@
-// gitm_vert_ensemble.hip -- the batch step kernel for one workgroup size.
+// gitm_vert_ensemble.hip -- the batch's Rusanov step kernel for one workgroup
+// size.
 //
 // Compiled once per size: GV_ENS_WAVES = 1..4 wavefronts per workgroup
 // (gitm_amd/build.py), each object defining launch_ensemble_w<GV_ENS_WAVES>
@@ -27,21 +28,21 @@ constexpr int NT = 64 * GV_ENS_WAVES;
 // checks that before it launches one.  Each member's RK4 carries live where
 // its table entry says (carry_lds), so that the members whose columns fit
 // the LDS budget of the tile keep them there and the others in scratch.
-template <int W, int SOLVER, bool IONS, class Ctx>
+template <int W, bool IONS, class Ctx>
 __device__ __forceinline__ void step_column(Ctx &cx, const gv::KParams &kp,
                                             const BatchMember &e, int col, double *lds,
                                             double dt) {
   if (e.carry_lds)
-    gv::run_column<64 * W, SOLVER, IONS, true>(cx, kp, e.io, col, lds, e.scratch, dt,
+    gv::run_column<64 * W, GITM_VERT_RUSANOV, IONS, true>(cx, kp, e.io, col, lds, e.scratch, dt,
                                                e.col_offset + col, e.io.n_alts,
                                                gv::scratch_fields(true, IONS));
   else
-    gv::run_column<64 * W, SOLVER, IONS, false>(cx, kp, e.io, col, lds, e.scratch, dt,
+    gv::run_column<64 * W, GITM_VERT_RUSANOV, IONS, false>(cx, kp, e.io, col, lds, e.scratch, dt,
                                                 e.col_offset + col, e.io.n_alts,
                                                 gv::scratch_fields(false, IONS));
 }
 
-template <int SOLVER, bool IONS>
+template <bool IONS>
 __global__ void __launch_bounds__(NT)
     vert_ensemble_kernel(gv::KParams kp, const BatchMember *__restrict__ mem, EnsLayout lay,
                          const double *__restrict__ dt_dev) {
@@ -70,7 +71,7 @@ __global__ void __launch_bounds__(NT)
         const double dt = dt_dev ? dt_dev[e.member] : kp.dt;
         GpuCtx cx{kp.err};
         if ((int)threadIdx.x < e.io.n_alts + 4)
-          step_column<NT / 64, SOLVER, IONS>(cx, kp, e, col, lds, dt);
+          step_column<NT / 64, IONS>(cx, kp, e, col, lds, dt);
       }
     }
     if (!tall) {
@@ -87,7 +88,7 @@ __global__ void __launch_bounds__(NT)
         const double dt = dt_dev ? dt_dev[e.member] : kp.dt;
         WaveCtx cx{{kp.err}, w << 6};
         if (cx.lane() < e.io.n_alts + 4)
-          step_column<1, SOLVER, IONS>(cx, kp, e, col, lds + (long long)w * lay.slot_doubles,
+          step_column<1, IONS>(cx, kp, e, col, lds + (long long)w * lay.slot_doubles,
                                        dt);
       }
     }
@@ -95,15 +96,9 @@ __global__ void __launch_bounds__(NT)
   }
 }
 
-template <int SOLVER, bool IONS>
-const void *kernel_of() {
-  return reinterpret_cast<const void *>(&vert_ensemble_kernel<SOLVER, IONS>);
-}
-
-const void *select_kernel(int solver, bool ions) {
-  if (solver == GITM_VERT_AUSM)
-    return ions ? kernel_of<GITM_VERT_AUSM, true>() : kernel_of<GITM_VERT_AUSM, false>();
-  return ions ? kernel_of<GITM_VERT_RUSANOV, true>() : kernel_of<GITM_VERT_RUSANOV, false>();
+const void *select_kernel(bool ions) {
+  return ions ? reinterpret_cast<const void *>(&vert_ensemble_kernel<true>)
+              : reinterpret_cast<const void *>(&vert_ensemble_kernel<false>);
 }
 
 }  // namespace
@@ -113,16 +108,16 @@ const void *select_kernel(int solver, bool ions) {
 
 // Workgroups of this size that one CU holds at once with `lds_bytes` of LDS
 // each (the persistent grid is that times the CU count); 0 on error.
-int GV_ENS_CAT(ensemble_occupancy_w, GV_ENS_WAVES)(int solver, bool ions, size_t lds_bytes) {
+int GV_ENS_CAT(ensemble_occupancy_w, GV_ENS_WAVES)(bool ions, size_t lds_bytes) {
   int n = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, select_kernel(solver, ions), NT,
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, select_kernel(ions), NT,
                                                    lds_bytes) != hipSuccess)
     return 0;
   return n;
 }
 
 // Queues one batch step: `grid` workgroups of NT threads, `lds_bytes` each.
-hipError_t GV_ENS_CAT(launch_ensemble_w, GV_ENS_WAVES)(int solver, bool ions, int grid,
+hipError_t GV_ENS_CAT(launch_ensemble_w, GV_ENS_WAVES)(bool ions, int grid,
                                                        size_t lds_bytes,
                                                        hipStream_t stream,
                                                        const gv::KParams &kp,
@@ -131,6 +126,6 @@ hipError_t GV_ENS_CAT(launch_ensemble_w, GV_ENS_WAVES)(int solver, bool ions, in
                                                        const double *dt_dev) {
   void *args[] = {const_cast<gv::KParams *>(&kp), &mem, const_cast<EnsLayout *>(&lay),
                   &dt_dev};
-  return hipLaunchKernel(select_kernel(solver, ions), dim3(grid), dim3(NT), args,
+  return hipLaunchKernel(select_kernel(ions), dim3(grid), dim3(NT), args,
                          lds_bytes, stream);
 }

@@ -23,6 +23,15 @@ struct GpuCtx {
   unsigned long long *err;
   __device__ int lane() const { return (int)threadIdx.x; }
   __device__ void sync() const { __syncthreads(); }
+  // x of the wavefront's first lane (for values that decide the same for all)
+  __device__ int uniform(int x) const { return __builtin_amdgcn_readfirstlane(x); }
+  // orders LDS writes before later reads by lanes of the same wavefront (see
+  // WaveCtx::sync)
+  __device__ void wave_sync() const {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+  }
   __device__ bool sync_or(bool p) const { return __syncthreads_or(p ? 1 : 0) != 0; }
   __device__ void report(unsigned long long key) const { atomicMin(err, key); }
   // Temp**DiffExp as exp(DiffExp*ln Temp): one log and six exp in place of
@@ -45,11 +54,7 @@ struct GpuCtx {
 struct WaveCtx : GpuCtx {
   int base;  // first thread of the wavefront
   __device__ int lane() const { return (int)threadIdx.x - base; }
-  __device__ void sync() const {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-  }
+  __device__ void sync() const { wave_sync(); }
   __device__ bool sync_or(bool p) const {
     sync();
     return __builtin_amdgcn_ballot_w64(p) != 0;

@@ -258,8 +258,9 @@ int gitm_vert_prepare(gitm_vert_handle *h, const gitm_vert_prep_params *p,
  * reference runs one model per MPI job and has no counterpart; each member
  * is stepped exactly as gitm_vert_advance would step it alone.
  *
- * A batch step is one launch over every member's columns, one lane per
- * level (see gitm_vert_batch_tile).  gitm_vert_batch_create builds the
+ * A batch step is one launch over the columns of every member of like height
+ * (AUSM: one to four launches), or of every member (Rusanov, see
+ * gitm_vert_batch_tile).  gitm_vert_batch_create builds the
  * device member table and reserves the scratch memory; afterwards
  * gitm_vert_batch_advance and gitm_vert_batch_prepare only queue kernels on
  * the handle's stream (no allocation, no copy, no synchronisation), so a
@@ -275,7 +276,9 @@ int gitm_vert_batch_create(gitm_vert_handle *h, const gitm_vert_columns *members
                            int n_members, int use_ion_advection, gitm_vert_batch **out);
 int gitm_vert_batch_destroy(gitm_vert_batch *b);
 
-/* Tile of a batch step.  Workgroups have waves_per_workgroup wavefronts
+/* Tile of a batch's Rusanov step (the AUSM step sizes its workgroups by the
+ * columns alone; a tile is checked and kept for it, and changes nothing).
+ * Workgroups have waves_per_workgroup wavefronts
  * (1..4, at least the tallest member's (nAlts+4)/64 rounded up).  A column of
  * more than 64 levels takes a whole workgroup; columns of at most 64 levels
  * take one wavefront each, columns_per_workgroup (1..waves_per_workgroup) of

@@ -5,19 +5,22 @@
 // (-1:0, n+1:n+2) held at their input values (the caller's message
 // exchange fills them, :20).
 //
-// Mapping: a workgroup takes APW altitudes of one block, a lane one cell of
-// one of them.  The workgroup stages the APW slices of every advected
-// variable (halo cells included) in LDS; each stage of the RK4 (:154-345)
-// then runs horizontal_solver (:535-818) lane by lane: the lane forms the
-// MC-limited face values of its own two faces in each direction
+// Mapping: a lane takes one cell of one altitude.  The workgroup stages the
+// slices of the advected variables (halo cells included) in LDS; each stage of
+// the RK4 (:154-345) then runs horizontal_solver (:535-818) lane by lane: the
+// lane forms the MC-limited face values of its own two faces in each direction
 // (calc_facevalues_lons/lats, :928-1034) from the slopes at its cell and
 // its two neighbours, the gradient and the Rusanov flux difference
 // (calc_rusanov_lons/lats, :821-922), and the updates, holding the new
-// values in registers until every lane has read the stage's state.  Every
+// values in registers until every lane has read the stage's state.  Density,
+// temperature and winds advance together; the species, whose equations read
+// the winds and nothing reads, are carried along.  Every
 // value is formed by the reference's operations in the reference's order,
 // so the results equal the reference's bit for bit (sin(latitude) aside,
 // which is the device's).  With UseImprovedIonAdvection a second kernel
 // applies the divergence of the ion velocity afterwards.
+#include <type_traits>
+
 #include "vert_gpu.h"
 
 namespace {
@@ -32,7 +35,6 @@ struct HzParams {
   int n_lons, n_lats, n_alts, n_blocks;
   int apw;         // altitudes per workgroup
   int alt_groups;  // workgroups per block
-  int k_first;     // the launch's first altitude
 };
 
 struct HzFields {
@@ -50,285 +52,542 @@ __device__ __forceinline__ double *hf(const gitm_vert_field &f, int lon, int lat
          (long long)b * f.s_blk;
 }
 
+// Limiter_mc (ModLimiter.f90:16-36) without branches: with both slopes of one
+// sign the smallest of beta |up|, beta |dn|, |up + dn| / 2 with that sign, else
+// zero.
 __device__ __forceinline__ double limiter(double beta, double up, double dn) {
-  // Limiter_mc (ModLimiter.f90:16-36)
-  if (up > 0.0) {
-    if (dn > 0.0) return fmin(fmin(beta * up, beta * dn), (up + dn) * 0.5);
-    return 0.0;
-  }
-  if (dn < 0.0) return fmax(fmax(beta * up, beta * dn), (up + dn) * 0.5);
-  return 0.0;
+  const double m = fmin(beta * fmin(fabs(up), fabs(dn)), fabs((up + dn) * 0.5));
+  const long long su = __builtin_bit_cast(long long, up), sd = __builtin_bit_cast(long long, dn);
+  return ((su ^ sd) < 0) ? 0.0 : __builtin_copysign(m, dn);
 }
 
 // The geometry of one cell i (1..n) along one line: InvD*Dist_FB at faces
-// i-1..i+2, d*Dist_FB at faces i and i+1, InvD*Dist_GB(i) and cMax at cells
-// i-1..i+1.
+// i-1..i+2, d*Dist_FB at faces i and i+1, InvD*Dist_GB(i), half the larger
+// cMax of the cells on either side of faces i and i+1, and whether the cell
+// is the line's first or last.
 struct LineGeo {
-  double ifb[4], dfb0, dfb1, igb, cm[3];
+  double ifb[4], dfb0, dfb1, igb, hc0, hc1;
+  bool first, last;
 };
 
-// One cell i (1..n) of one line: v(m) = Var(i + m), m = -3..3 (the line's
-// cells -1..n+2 only).  Returns the gradient and the flux difference.
-template <class VF>
-__device__ __forceinline__ void rusanov_cell(int i, int n, VF v, const LineGeo &g,
-                                             double beta, double &grad, double &diff) {
-  auto ifb = [&](int m) { return g.ifb[m + 1]; };
-  const double dfb0 = g.dfb0, dfb1 = g.dfb1, igb = g.igb, cmm = g.cm[0], cm0 = g.cm[1],
-               cmp = g.cm[2];
+// One cell of one line: v[m * S] = Var(i + m), m = -3..3.  Gradient and flux
+// difference (calc_facevalues_lons/lats, calc_rusanov_lons/lats).  The slope
+// of a cell takes the fourth-order difference of its two faces; a face's is
+// the same seen from either cell, so the three slopes need four.  The faces
+// beyond the line's outermost slopes take the plain difference; there m = -3
+// or 3 lies outside the line, is read from whatever the LDS holds and not
+// used.
+template <class P>
+__device__ __forceinline__ void rusanov_cell(const P v, int S, const LineGeo &g, double beta,
+                                             double &grad, double &diff) {
   const double F1 = 0.6250000, F2 = 0.0416667;
-  double dl[3];
-#pragma unroll
-  for (int t = 0; t < 3; t++) {  // slopes at cells i-1, i, i+1
-    const int m = t - 1, c = i + m;
-    double up, dn;
-    if (c <= n) {
-      const double h = ifb(m + 1) * 2;
-      up = h * (F1 * (v(m + 1) - v(m)) - F2 * (v(m + 2) - v(m - 1)));
-    } else {
-      up = (v(m + 1) - v(m)) * ifb(m + 1);
-    }
-    if (c >= 1) {
-      const double h = ifb(m) * 2;
-      dn = h * (F1 * (v(m) - v(m - 1)) - F2 * (v(m + 1) - v(m - 2)));
-    } else {
-      dn = (v(m) - v(m - 1)) * ifb(m);
-    }
-    dl[t] = limiter(beta, up, dn);
-  }
-  const double l0 = v(-1) + 0.5 * dl[0] * dfb0, r0 = v(0) - 0.5 * dl[1] * dfb0;
-  const double l1 = v(0) + 0.5 * dl[1] * dfb1, r1 = v(1) - 0.5 * dl[2] * dfb1;
-  const double f0 = 0.5 * fmax(cmm, cm0) * (r0 - l0);
-  const double f1 = 0.5 * fmax(cm0, cmp) * (r1 - l1);
-  grad = 0.5 * (l1 + r1 - l0 - r0) * igb;
-  diff = (f1 - f0) * igb;
+  const double vm3 = v[-3 * S], vm2 = v[-2 * S], vm1 = v[-S], v0 = v[0], v1 = v[S],
+               v2 = v[2 * S], v3 = v[3 * S];
+  const double dm = vm1 - vm2, dp = v2 - v1;
+  double f0 = (g.ifb[0] * 2) * (F1 * dm - F2 * (v0 - vm3));
+  const double f1 = (g.ifb[1] * 2) * (F1 * (v0 - vm1) - F2 * (v1 - vm2));
+  const double f2 = (g.ifb[2] * 2) * (F1 * (v1 - v0) - F2 * (v2 - vm1));
+  double f3 = (g.ifb[3] * 2) * (F1 * dp - F2 * (v3 - v0));
+  f0 = g.first ? dm * g.ifb[0] : f0;
+  f3 = g.last ? dp * g.ifb[3] : f3;
+  const double s0 = limiter(beta, f1, f0), s1 = limiter(beta, f2, f1), s2 = limiter(beta, f3, f2);
+  const double l0 = vm1 + 0.5 * s0 * g.dfb0, r0 = v0 - 0.5 * s1 * g.dfb0;
+  const double l1 = v0 + 0.5 * s1 * g.dfb1, r1 = v1 - 0.5 * s2 * g.dfb1;
+  grad = 0.5 * (l1 + r1 - l0 - r0) * g.igb;
+  diff = (g.hc1 * (r1 - l1) - g.hc0 * (r0 - l0)) * g.igb;
 }
 
-// (256 lanes at most; two wavefronts per SIMD: the LDS of three workgroups
-// per CU holds about that many anyway).  TOPO: UseTopography, launched for
-// one altitude at a time (the host walks k = 1..nAlts), so that the level
-// below already holds the step's result when dVarDAlt reads it.
+// The advected fields (advance_horizontal.f90:154-167) by number.
+__device__ __forceinline__ const gitm_vert_field &hz_field(const gitm_vert_columns &io, int v,
+                                                           int &comp) {
+  if (v == V_RHO) { comp = 0; return io.rho; }
+  if (v == V_TEMP) { comp = 0; return io.temperature; }
+  if (v < V_NUM) { comp = v - V_VEL; return io.velocity; }
+  if (v < V_VV) { comp = v - V_NUM; return io.ndensity_s; }
+  if (v < V_INUM) { comp = v - V_VV; return io.vertical_velocity; }
+  comp = v - V_INUM;
+  return io.idensity_s;
+}
+
+// One lane's cell of one altitude: its geometry, and what the core's four
+// stages leave for the other variables.
+struct HzCell {
+  int i, jl, k, b;
+  LineGeo lo, la;
+  double hz, slon, slat;     // UseTopography: 0.5 / dAlt_GB, the surface's slopes
+  double ve[4], vn[4], div[4];
+};
+
+__device__ __forceinline__ double at_stage(const double (&x)[4], int s) {
+  return s == 0 ? x[0] : s == 1 ? x[1] : s == 2 ? x[2] : x[3];
+}
+__device__ __forceinline__ void set_stage(double (&x)[4], int s, double v) {
+  x[0] = s == 0 ? v : x[0];
+  x[1] = s == 1 ? v : x[1];
+  x[2] = s == 2 ? v : x[2];
+  x[3] = s == 3 ? v : x[3];
+}
+
+template <bool TOPO>
+__device__ __forceinline__ void hz_geometry(HzCell &c, const gitm_vert_columns &io,
+                                            const HzFields &f, int nlo, int nla) {
+  const int i = c.i, jl = c.jl, k = c.k, b = c.b;
+#pragma unroll
+  for (int m = -1; m <= 2; m++) {
+    c.lo.ifb[m + 1] = *hf(f.inv_dlon_fb, i + m, jl, k, 0, b);
+    c.la.ifb[m + 1] = *hf(f.inv_dlat_fb, i, jl + m, k, 0, b);
+  }
+  c.lo.dfb0 = *hf(f.dlon_fb, i, jl, k, 0, b);
+  c.lo.dfb1 = *hf(f.dlon_fb, i + 1, jl, k, 0, b);
+  c.la.dfb0 = *hf(f.dlat_fb, i, jl, k, 0, b);
+  c.la.dfb1 = *hf(f.dlat_fb, i, jl + 1, k, 0, b);
+  c.lo.igb = *hf(f.inv_dlon_gb, i, jl, k, 0, b);
+  c.la.igb = *hf(f.inv_dlat_gb, i, jl, k, 0, b);
+  const double o0 = *hf(f.cmax, i, jl, k, 0, b), a0 = *hf(f.cmax, i, jl, k, 1, b);
+  c.lo.hc0 = 0.5 * fmax(*hf(f.cmax, i - 1, jl, k, 0, b), o0);
+  c.lo.hc1 = 0.5 * fmax(o0, *hf(f.cmax, i + 1, jl, k, 0, b));
+  c.la.hc0 = 0.5 * fmax(*hf(f.cmax, i, jl - 1, k, 1, b), a0);
+  c.la.hc1 = 0.5 * fmax(a0, *hf(f.cmax, i, jl + 1, k, 1, b));
+  c.lo.first = i == 1;
+  c.lo.last = i == nlo;
+  c.la.first = jl == 1;
+  c.la.last = jl == nla;
+  if (TOPO) {
+    // 0.5 / dAlt and the slopes of the level surface (advance_horizontal.f90
+    // :581-582, :870-871, :919-920)
+    c.hz = 0.5 / *hf(f.dalt, i, jl, k, 0, b);
+    c.slon = *hf(f.dalt_dlon, i, jl, k, 0, b);
+    c.slat = *hf(f.dalt_dlat, i, jl, k, 0, b);
+  }
+}
+
+// The RK4 bookkeeping of one variable (:184-345): the stage's new value nw
+// and state x give the next stage's state (the last stage's: the result).
+__device__ __forceinline__ double hz_rk(int stage, double nw, double x, double orig,
+                                        double &acc) {
+  const double K = nw - x;
+  if (stage == 3) return orig + (1.0 / 6.0) * (acc + K);
+  acc = stage == 0 ? K : acc + 2.0 * K;
+  return (stage == 2 ? K : 0.5 * K) + orig;
+}
+
+constexpr int NCORE = 5;  // Rho, Temperature and the winds advance together
+
+// Grad and Diff of one variable in both directions (:588-662); dz: the
+// variable's 0.5 (Var(k+1) - Var(k-1)) / dAlt (:583-586)
+template <bool TOPO>
+__device__ __forceinline__ void hz_gd(const HzCell &c, const double *x, int NLo, double beta,
+                                      double dz, double &glon, double &glat, double &dsum) {
+  double dlon, dlat;
+  rusanov_cell(x, 1, c.lo, beta, glon, dlon);
+  GV_ORDER();
+  rusanov_cell(x, NLo, c.la, beta, glat, dlat);
+  if (TOPO) {
+    glon = glon - dz * c.slon;
+    glat = glat - dz * c.slat;
+  }
+  dsum = dlon + dlat;
+  GV_HERE(glon);
+  GV_HERE(glat);
+  GV_HERE(dsum);
+  GV_ORDER();
+}
+
+// New values (:667-816) of the core variables from the stage's state, the
+// gradients and the flux differences.
+__device__ __forceinline__ void hz_core_update(const HzParams &p, const double (&g)[6],
+                                               double rho, double tmp, double ve, double vn,
+                                               double vu, double div, const double (&go)[NCORE],
+                                               const double (&ga)[NCORE],
+                                               const double (&d)[NCORE], double (&nw)[NCORE]) {
+  constexpr int E = V_VEL, N = V_VEL + 1, U = V_VEL + 2;
+  const double dt = p.dt;
+  const double invr = g[0], rd = g[1], gam = g[2], tl = g[3], cosl = g[4], sinl = g[5];
+  const double csin = sinl * 2 * p.omega, ccos = cosl * 2 * p.omega;
+  const double cent = p.omega * p.omega * cosl * sinl;
+  nw[V_RHO] = rho - dt * (rho * div + ga[V_RHO] * vn + go[V_RHO] * ve) + dt * d[V_RHO];
+  double we = ve -
+              dt * (vn * ga[E] + ve * go[E] + ve * (vu - tl * vn) * invr + go[V_TEMP] +
+                    go[V_RHO] * tmp / rho) +
+              dt * d[E];
+  double wn = vn -
+              dt * (vn * ga[N] + ve * go[N] + (vn * vu + tl * (ve * ve)) * invr + ga[V_TEMP] +
+                    ga[V_RHO] * tmp / rho) +
+              dt * d[N];
+  if (p.use_coriolis) {
+    we = we + dt * (+csin * vn - ccos * vu);
+    wn = wn - dt * (cent * rd + csin * ve);
+  }
+  nw[E] = we;
+  nw[N] = wn;
+  nw[V_TEMP] =
+      tmp - dt * ((gam - 1) * tmp * div + ga[V_TEMP] * vn + go[V_TEMP] * ve) + dt * d[V_TEMP];
+  nw[U] = vu - dt * (vn * ga[U] + ve * go[U]) + dt * d[U];
+}
+
+// New value of one of the variables that the core carries along: 0 NDensityS,
+// 1 VerticalVelocity, 2 IDensityS (with the ion velocity in ve, vn).
+template <int KIND>
+__device__ __forceinline__ double hz_carried_update(double q, double dt, double go, double ga,
+                                                    double d, double ve, double vn, double div) {
+  if (KIND == 0) return q - dt * (q * div + ga * vn + go * ve) + dt * d;
+  if (KIND == 1) return q - dt * (vn * ga + ve * go) + dt * d;
+  return q - dt * (+ga * vn + go * ve) + dt * d;
+}
+
+// Per-cell inputs of the core's updates.
+__device__ __forceinline__ void hz_cell_inputs(const HzCell &c, const gitm_vert_columns &io,
+                                               const HzFields &f, double (&g)[6]) {
+  g[0] = *hf(io.inv_radial_distance, c.i, c.jl, c.k, 0, c.b);
+  g[1] = *hf(f.raddist, c.i, c.jl, c.k, 0, c.b);
+  g[2] = *hf(io.gamma, c.i, c.jl, c.k, 0, c.b);
+  g[3] = *hf(f.tan_latitude, 1, c.jl, 0, 0, c.b);
+  g[4] = *hf(io.cos_latitude, 1, c.jl, 0, 0, c.b);
+  g[5] = sin(*hf(f.latitude, 1, c.jl, 0, 0, c.b));
+}
+
+// Write back (:349-429).
+__device__ __forceinline__ void hz_store_core(const HzCell &c, const gitm_vert_columns &io,
+                                              const HzFields &f, const double (&u)[NCORE],
+                                              double told) {
+  *hf(io.rho, c.i, c.jl, c.k, 0, c.b) = u[V_RHO];
+#pragma unroll
+  for (int q = 0; q < 3; q++) *hf(io.velocity, c.i, c.jl, c.k, q, c.b) = u[V_VEL + q];
+  if (f.temp_source.ptr) *hf(f.temp_source, c.i, c.jl, c.k, 0, c.b) = u[V_TEMP] - told;
+  *hf(io.temperature, c.i, c.jl, c.k, 0, c.b) = u[V_TEMP];
+}
+__device__ __forceinline__ void hz_report(const HzCell &c, int nlo, int nla,
+                                          unsigned long long *err) {
+  const int column = (c.b * nla + (c.jl - 1)) * nlo + (c.i - 1);
+  atomicMin(err, gv::error_key(column, GITM_VERT_ENONPOSITIVE, c.k));
+}
+// The floored advected ion (:405-417) s of the cell.
+__device__ __forceinline__ double hz_store_ion(const HzCell &c, const gitm_vert_columns &io,
+                                               int s, double v) {
+  if (v < 1.0e2) v = 1.0e2;
+  *hf(io.idensity_s, c.i, c.jl, c.k, s, c.b) = v;
+  return v;
+}
+__device__ __forceinline__ void hz_store_electrons(const HzCell &c,
+                                                   const gitm_vert_columns &io) {
+  double e = 0.0;  // :420-425
+  for (int s = 0; s < gv::NIONS - 1; s++)
+    e = e + *hf(io.idensity_s, c.i, c.jl, c.k, s, c.b);
+  *hf(io.idensity_s, c.i, c.jl, c.k, gv::NIONS - 1, c.b) = e;
+}
+
+// LDS doubles before the first and after the last slice: the reads of m = -3
+// and 3 past a line's end stay inside the block.
+__host__ __device__ constexpr int hz_pad(int nlo) { return nlo + 4 + 4; }
+
+// ---------------------------------------------------------------------------
+// Level surfaces (no UseTopography): the altitudes are independent.  A
+// workgroup takes apw altitudes of one block, a lane one cell of one of them.
+// The core variables run their four stages first (:154-345); the others do
+// not feed back on them, so they follow in groups that reuse the same LDS
+// slices, with the core's winds and divergence of each stage kept in
+// registers, as are the RK4's starting values and sums.
+// Six slices per altitude instead of seventeen and their new values, so that
+// the lanes can be packed (three 9x9 altitudes on 243 of 256 lanes) and three
+// wavefronts share a SIMD.  FP64 issue bounds it: 800 blocks of 9x9 x 100
+// levels, 8.8 -> 3.1 ms (all variables at once, one altitude on 81 of 128
+// lanes, the RK4 sums and starting values in device memory, six face
+// differences per cell and direction before).  Three wavefronts per SIMD (168
+// registers, no spills) against four (128, 42 spilled): 3.1 against 3.5 ms.
 // BLON, BLAT: the block's cells per direction when fixed at compile time
 // (GITM's are, 9 x 9 by default), so that the LDS and cell indexing is
 // constant; 0 takes them from the parameters.
-template <int NV, bool TOPO, int BLON = 0, int BLAT = 0>
-__global__ void __launch_bounds__(256, 2)
-    horiz_kernel(HzParams p, gitm_vert_columns io, HzFields f, unsigned long long *err,
-                 double *accg) {
+// ---------------------------------------------------------------------------
+constexpr int HZ_GROUP = 6;
+
+template <bool IONS, int BLON, int BLAT>
+__global__ void __launch_bounds__(256, 3)
+    horiz_flat_kernel(HzParams p, gitm_vert_columns io, HzFields f, unsigned long long *err) {
   extern __shared__ double lds[];
   const int nlo = BLON ? BLON : p.n_lons, nla = BLAT ? BLAT : p.n_lats, NLo = nlo + 4,
             NLg = nla + 4;
-  const int cells = nlo * nla, slab = NV * NLg * NLo;
-  const int b = (int)blockIdx.x / p.alt_groups;
-  const int k0 = p.k_first + ((int)blockIdx.x % p.alt_groups) * p.apw;
+  const int cells = nlo * nla, plane = NLg * NLo;
+  const int k0 = 1 + ((int)blockIdx.x % p.alt_groups) * p.apw;
   const int napw = min(p.apw, p.n_alts - k0 + 1);
-  const int tid = (int)threadIdx.x;
-  const int a = tid / cells, cell = tid % cells;
+  const int tid = (int)threadIdx.x, a = tid / cells, cell = tid % cells;
   const bool active = a < napw;
-  const int i = cell % nlo + 1, jl = cell / nlo + 1, k = k0 + a;
-  // the advected fields (advance_horizontal.f90:154-167)
-  auto field = [&](int v, int &comp) -> const gitm_vert_field & {
-    if (v == V_RHO) { comp = 0; return io.rho; }
-    if (v == V_TEMP) { comp = 0; return io.temperature; }
-    if (v < V_NUM) { comp = v - V_VEL; return io.velocity; }
-    if (v < V_VV) { comp = v - V_NUM; return io.ndensity_s; }
-    if (v < V_INUM) { comp = v - V_VV; return io.vertical_velocity; }
-    comp = v - V_INUM;
-    return io.idensity_s;
-  };
-  // stage the slices: x[a][v][lat][lon], halo cells included; after the
-  // slices, per altitude, the stage's new values, [v][cell].  The RK4 sums
-  // live in device memory (accg, [workgroup][altitude][v][cell]): they are
-  // touched once per stage, and the LDS they would take costs a workgroup
-  // per CU.
-  // Each thread takes the cells r2 = tid, tid + blockDim.x, .. of a slice
-  // (two at most: a slice has (nla+4)(nlo+4) cells) and stages them for
-  // every variable and altitude, so that the only integer divisions are the
-  // per-cell ones, not one per element.
-  {
-    const int plane = NLg * NLo;
+  HzCell c;
+  c.b = (int)blockIdx.x / p.alt_groups;
+  c.i = cell % nlo + 1;
+  c.jl = cell / nlo + 1;
+  c.k = k0 + (active ? a : 0);
+  double *const slices = lds + hz_pad(nlo);
+  double *const x = slices + (active ? a : 0) * HZ_GROUP * plane + (c.jl + 1) * NLo + c.i + 1;
+  // variables v0..v0+n-1, halo cells included: [altitude][variable][lat][lon];
+  // each thread takes the cells r2 = tid, tid + 256, .. of a slice
+  auto stage_in = [&](int v0, int n) {
     for (int r2 = tid; r2 < plane; r2 += (int)blockDim.x) {
       const int lat = r2 / NLo - 1, lon = r2 % NLo - 1;
       for (int aa = 0; aa < napw; aa++) {
+        double *d = slices + aa * HZ_GROUP * plane + r2;
 #pragma unroll
-        for (int v = 0; v < NV; v++) {
-          int comp;
-          const gitm_vert_field &g = field(v, comp);
-          lds[(aa * NV + v) * plane + r2] = *hf(g, lon, lat, k0 + aa, comp, b);
-        }
+        for (int v = 0; v < HZ_GROUP; v++)
+          if (v < n) {
+            int comp;
+            const gitm_vert_field &g = hz_field(io, v0 + v, comp);
+            d[v * plane] = *hf(g, lon, lat, k0 + aa, comp, c.b);
+          }
       }
     }
-  }
-  const int aw = active ? a : 0;
-  double *x = lds + (long long)aw * slab;
-  double *nwb = lds + (long long)p.apw * slab + (long long)aw * NV * cells;
-  double *accb = accg + ((long long)blockIdx.x * p.apw + aw) * NV * cells;
-  auto X = [&](int v, int lat, int lon) -> double & {
-    return x[(v * NLg + lat + 1) * NLo + lon + 1];
   };
-  auto NW = [&](int v) -> double & { return nwb[v * cells + cell]; };
-  auto ACC = [&](int v) -> double & { return accb[v * cells + cell]; };
+  stage_in(V_RHO, NCORE);
+  double g[6];
+  if (active) {
+    hz_geometry<false>(c, io, f, nlo, nla);
+    hz_cell_inputs(c, io, f, g);
+  }
   __syncthreads();
-  // per-cell inputs of the updates
-  double invr = 0, rd = 0, gam = 0, tl = 0, cosl = 0, sinl = 0, ive = 0, ivn = 0;
-  if (active) {
-    invr = *hf(io.inv_radial_distance, i, jl, k, 0, b);
-    rd = *hf(f.raddist, i, jl, k, 0, b);
-    gam = *hf(io.gamma, i, jl, k, 0, b);
-    tl = *hf(f.tan_latitude, 1, jl, 0, 0, b);
-    cosl = *hf(io.cos_latitude, 1, jl, 0, 0, b);
-    sinl = sin(*hf(f.latitude, 1, jl, 0, 0, b));
-    if (NV == NV_IONS) {
-      ive = *hf(io.ivelocity, i, jl, k, 0, b);
-      ivn = *hf(io.ivelocity, i, jl, k, 1, b);
-    }
-  }
-  LineGeo glo{}, gla{};
-  if (active) {
+  {
+    double orig[NCORE], acc[NCORE];
 #pragma unroll
-    for (int m = -1; m <= 2; m++) {
-      glo.ifb[m + 1] = *hf(f.inv_dlon_fb, i + m, jl, k, 0, b);
-      gla.ifb[m + 1] = *hf(f.inv_dlat_fb, i, jl + m, k, 0, b);
-    }
-    glo.dfb0 = *hf(f.dlon_fb, i, jl, k, 0, b);
-    glo.dfb1 = *hf(f.dlon_fb, i + 1, jl, k, 0, b);
-    gla.dfb0 = *hf(f.dlat_fb, i, jl, k, 0, b);
-    gla.dfb1 = *hf(f.dlat_fb, i, jl + 1, k, 0, b);
-    glo.igb = *hf(f.inv_dlon_gb, i, jl, k, 0, b);
-    gla.igb = *hf(f.inv_dlat_gb, i, jl, k, 0, b);
+    for (int v = 0; v < NCORE; v++) orig[v] = x[v * plane];
+    double u[NCORE];
+#pragma unroll 1
+    for (int stage = 0; stage < 4; stage++) {
+      if (active) {
+        double go[NCORE], ga[NCORE], d[NCORE];
 #pragma unroll
-    for (int m = -1; m <= 1; m++) {
-      glo.cm[m + 1] = *hf(f.cmax, i + m, jl, k, 0, b);
-      gla.cm[m + 1] = *hf(f.cmax, i, jl + m, k, 1, b);
-    }
-  }
-  // UseTopography: 0.5 / dAlt and the slopes of the level surface
-  // (advance_horizontal.f90:581-582, :870-871, :919-920)
-  double hz = 0, slon = 0, slat = 0;
-  if (TOPO && active) {
-    hz = 0.5 / *hf(f.dalt, i, jl, k, 0, b);
-    slon = *hf(f.dalt_dlon, i, jl, k, 0, b);
-    slat = *hf(f.dalt_dlat, i, jl, k, 0, b);
-  }
-  const double dt = p.dt, om = p.omega;
-  const double csin = sinl * 2 * om, ccos = cosl * 2 * om;
-  const double cent = om * om * cosl * sinl;
-
-#pragma unroll 1
-  for (int stage = 0; stage < 4; stage++) {
-    if (active) {
-      // Grad and Diff of variable v in both directions (:588-662)
-      auto gd = [&](int v, double &glon, double &dlon, double &glat, double &dlat) {
-        rusanov_cell(i, nlo, [&](int m) { return X(v, jl, i + m); }, glo, p.beta, glon, dlon);
-        rusanov_cell(jl, nla, [&](int m) { return X(v, jl + m, i); }, gla, p.beta, glat, dlat);
-        if (TOPO) {  // dVarDAlt_C from the state arrays (:583-586, :591-662)
-          int comp;
-          const gitm_vert_field &g = field(v, comp);
-          const double dz = hz * (*hf(g, i, jl, k + 1, comp, b) - *hf(g, i, jl, k - 1, comp, b));
-          glon = glon - dz * slon;
-          glat = glat - dz * slat;
+        for (int v = 0; v < NCORE; v++)
+          hz_gd<false>(c, x + v * plane, NLo, p.beta, 0.0, go[v], ga[v], d[v]);
+        const double ve = x[V_VEL * plane], vn = x[(V_VEL + 1) * plane];
+        const double div = ga[V_VEL + 1] + go[V_VEL] - g[3] * vn * g[0];
+        set_stage(c.ve, stage, ve);
+        set_stage(c.vn, stage, vn);
+        set_stage(c.div, stage, div);
+        hz_core_update(p, g, x[V_RHO * plane], x[V_TEMP * plane], ve, vn,
+                       x[(V_VEL + 2) * plane], div, go, ga, d, u);
+      }
+      __syncthreads();  // every lane has read the stage's state
+      if (active)
+#pragma unroll
+        for (int v = 0; v < NCORE; v++) {
+          u[v] = hz_rk(stage, u[v], x[v * plane], orig[v], acc[v]);
+          x[v * plane] = u[v];
         }
-      };
-      const double rho = X(V_RHO, jl, i), tmp = X(V_TEMP, jl, i);
-      const double ve = X(V_VEL + 0, jl, i), vn = X(V_VEL + 1, jl, i), vu = X(V_VEL + 2, jl, i);
-      double gE[4], gN[4], gU[4], gR[4], gT[4];  // glon, dlon, glat, dlat
-      gd(V_VEL + 0, gE[0], gE[1], gE[2], gE[3]);
-      gd(V_VEL + 1, gN[0], gN[1], gN[2], gN[3]);
-      const double div = gN[2] + gE[0] - tl * vn * invr;
-      gd(V_RHO, gR[0], gR[1], gR[2], gR[3]);
-      gd(V_TEMP, gT[0], gT[1], gT[2], gT[3]);
-      // the updates (:667-816), New starting from the stage's state
-      NW(V_RHO) = rho - dt * (rho * div + gR[2] * vn + gR[0] * ve) + dt * (gR[1] + gR[3]);
-      double we = ve -
-                  dt * (vn * gE[2] + ve * gE[0] + ve * (vu - tl * vn) * invr + gT[0] +
-                        gR[0] * tmp / rho) +
-                  dt * (gE[1] + gE[3]);
-      double wn = vn -
-                  dt * (vn * gN[2] + ve * gN[0] + (vn * vu + tl * (ve * ve)) * invr + gT[2] +
-                        gR[2] * tmp / rho) +
-                  dt * (gN[1] + gN[3]);
-      if (p.use_coriolis) {
-        we = we + dt * (+csin * vn - ccos * vu);
-        wn = wn - dt * (cent * rd + csin * ve);
-      }
-      NW(V_VEL + 0) = we;
-      NW(V_VEL + 1) = wn;
-      NW(V_TEMP) = tmp - dt * ((gam - 1) * tmp * div + gT[2] * vn + gT[0] * ve) +
-                   dt * (gT[1] + gT[3]);
-      gd(V_VEL + 2, gU[0], gU[1], gU[2], gU[3]);
-      NW(V_VEL + 2) = vu - dt * (vn * gU[2] + ve * gU[0]) + dt * (gU[1] + gU[3]);
-#pragma unroll 1
-      for (int v = V_NUM; v < NV; v++) {
-        double g0, g1, g2, g3;
-        gd(v, g0, g1, g2, g3);
-        const double q = X(v, jl, i);
-        double w;
-        if (v < V_VV)  // NDensityS
-          w = q - dt * (q * div + g2 * vn + g0 * ve) + dt * (g1 + g3);
-        else if (v < V_INUM)  // VerticalVelocity
-          w = q - dt * (vn * g2 + ve * g0) + dt * (g3 + g1);
-        else  // IDensityS(1:nIonsAdvect), carried by the ion velocity
-          w = q - dt * (+g2 * ivn + g0 * ive) + dt * (g1 + g3);
-        NW(v) = w;
-      }
+      __syncthreads();
     }
-    __syncthreads();  // every lane has read the stage's state
-    if (active) {
-      // the RK4 bookkeeping (:184-345)
-#pragma unroll 1
-      for (int v = 0; v < NV; v++) {
-        int comp;
-        const double orig = *hf(field(v, comp), i, jl, k, comp, b);
-        const double K = NW(v) - X(v, jl, i);
-        double u;
-        if (stage == 0) {
-          ACC(v) = K;
-          u = 0.5 * K + orig;
-        } else if (stage == 1) {
-          ACC(v) = ACC(v) + 2.0 * K;
-          u = 0.5 * K + orig;
-        } else if (stage == 2) {
-          ACC(v) = ACC(v) + 2.0 * K;
-          u = K + orig;
-        } else {
-          const double sum = ACC(v) + K;
-          u = orig + (1.0 / 6.0) * sum;
-        }
-        X(v, jl, i) = u;
-      }
+    if (active) hz_store_core(c, io, f, u, orig[V_TEMP]);
+  }
+  auto carried = [&](auto kind, int v0, auto count, auto &&store) {
+    constexpr int KIND = decltype(kind)::value, N = decltype(count)::value;
+    stage_in(v0, N);
+    double ive = 0.0, ivn = 0.0;
+    if (KIND == 2 && active) {
+      ive = *hf(io.ivelocity, c.i, c.jl, c.k, 0, c.b);
+      ivn = *hf(io.ivelocity, c.i, c.jl, c.k, 1, c.b);
     }
     __syncthreads();
-  }
-  if (!active) return;
-  // write back (:349-429)
-  bool negative = false;
+    double orig[N], acc[N], u[N];
 #pragma unroll
-  for (int s = 0; s < gv::NSP; s++) negative = negative || X(V_NUM + s, jl, i) < 0.0;
-  if (negative) {
-    const int column = (b * nla + (jl - 1)) * nlo + (i - 1);
-    atomicMin(err, gv::error_key(column, GITM_VERT_ENONPOSITIVE, k));
-  }
-  const double told = *hf(io.temperature, i, jl, k, 0, b);
-  *hf(io.rho, i, jl, k, 0, b) = X(V_RHO, jl, i);
+    for (int v = 0; v < N; v++) orig[v] = x[v * plane];
+#pragma unroll 1
+    for (int stage = 0; stage < 4; stage++) {
+      if (active) {
+        const double ve = KIND == 2 ? ive : at_stage(c.ve, stage),
+                     vn = KIND == 2 ? ivn : at_stage(c.vn, stage), div = at_stage(c.div, stage);
 #pragma unroll
-  for (int c = 0; c < 3; c++) *hf(io.velocity, i, jl, k, c, b) = X(V_VEL + c, jl, i);
-  if (f.temp_source.ptr) *hf(f.temp_source, i, jl, k, 0, b) = X(V_TEMP, jl, i) - told;
-  *hf(io.temperature, i, jl, k, 0, b) = X(V_TEMP, jl, i);
+        for (int v = 0; v < N; v++) {
+          double go, ga, d;
+          hz_gd<false>(c, x + v * plane, NLo, p.beta, 0.0, go, ga, d);
+          u[v] = hz_carried_update<KIND>(x[v * plane], p.dt, go, ga, d, ve, vn, div);
+          GV_HERE(u[v]);
+          GV_ORDER();
+        }
+      }
+      __syncthreads();
+      if (active)
 #pragma unroll
-  for (int s = 0; s < gv::NSP; s++) {
-    *hf(io.vertical_velocity, i, jl, k, s, b) = X(V_VV + s, jl, i);
-    *hf(io.ndensity_s, i, jl, k, s, b) = X(V_NUM + s, jl, i);
-  }
-  if (NV == NV_IONS) {
-#pragma unroll
-    for (int s = 0; s < NIA; s++) {
-      double v = X(V_INUM + s, jl, i);
-      if (v < 1.0e2) v = 1.0e2;  // :405-417
-      *hf(io.idensity_s, i, jl, k, s, b) = v;
+        for (int v = 0; v < N; v++) {
+          u[v] = hz_rk(stage, u[v], x[v * plane], orig[v], acc[v]);
+          x[v * plane] = u[v];
+        }
+      __syncthreads();
     }
-    double e = 0.0;  // electrons, :420-425
-    for (int s = 0; s < gv::NIONS - 1; s++) e = e + *hf(io.idensity_s, i, jl, k, s, b);
-    *hf(io.idensity_s, i, jl, k, gv::NIONS - 1, b) = e;
+    if (active) store(u);
+  };
+  carried(std::integral_constant<int, 0>(), V_NUM, std::integral_constant<int, gv::NSP>(),
+          [&](const double (&u)[gv::NSP]) {
+            bool negative = false;
+#pragma unroll
+            for (int s = 0; s < gv::NSP; s++) {
+              negative = negative || u[s] < 0.0;
+              *hf(io.ndensity_s, c.i, c.jl, c.k, s, c.b) = u[s];
+            }
+            if (negative) hz_report(c, nlo, nla, err);
+          });
+  carried(std::integral_constant<int, 1>(), V_VV, std::integral_constant<int, gv::NSP>(),
+          [&](const double (&u)[gv::NSP]) {
+#pragma unroll
+            for (int s = 0; s < gv::NSP; s++)
+              *hf(io.vertical_velocity, c.i, c.jl, c.k, s, c.b) = u[s];
+          });
+  if (IONS)
+    carried(std::integral_constant<int, 2>(), V_INUM, std::integral_constant<int, NIA>(),
+            [&](const double (&u)[NIA]) {
+#pragma unroll
+              for (int s = 0; s < NIA; s++) hz_store_ion(c, io, s, u[s]);
+              hz_store_electrons(c, io);
+            });
+}
+
+// ---------------------------------------------------------------------------
+// UseTopography: dVarDAlt reads the level below as the step leaves it and the
+// level above as it was (:583-586), so a block's levels follow one another.
+// One workgroup walks a block's levels: no launch per level, and the chain of
+// levels is shortened by giving the variables to teams of wavefronts that
+// work side by side.  Team 0 takes the core variables, the others VP of the
+// carried ones each (the ions' team the two ions); all have the cells of the
+// level.  In each stage the teams form their gradients, the core's team puts
+// its winds and divergence in LDS, and after a barrier every team updates.
+// The chain of levels bounds it where blocks are few: 32 blocks of 9x9 x 50
+// levels with ions 6.45 -> 1.5 ms (one launch per level before).
+// A lane keeps its own cell's result for the level above.
+// ---------------------------------------------------------------------------
+enum { TEAM_CORE = 0, TEAM_DENSITY, TEAM_WIND, TEAM_ION };
+
+template <int KIND, int N, int BLON, int BLAT>
+__device__ __forceinline__ void topo_team(const HzParams &p, const gitm_vert_columns &io,
+                                          const HzFields &f, unsigned long long *err,
+                                          double *slices, double *pub, int cell,
+                                          int team_threads, int s0) {
+  const int nlo = BLON ? BLON : p.n_lons, nla = BLAT ? BLAT : p.n_lats, NLo = nlo + 4,
+            NLg = nla + 4;
+  const int cells = nlo * nla, plane = NLg * NLo;
+  constexpr int V0 = KIND == TEAM_CORE ? V_RHO : KIND == TEAM_DENSITY ? V_NUM
+                     : KIND == TEAM_WIND ? V_VV : V_INUM;
+  const bool active = cell < cells;
+  HzCell c;
+  c.b = (int)blockIdx.x;
+  c.i = active ? cell % nlo + 1 : 1;
+  c.jl = active ? cell / nlo + 1 : 1;
+  double *const mine = slices + (V0 + s0) * plane;
+  double *const x = mine + (c.jl + 1) * NLo + c.i + 1;
+  // a variable of the team at (lon, lat, k)
+  const auto at = [&](int v, int lon, int lat, int k) -> double * {
+    if (KIND == TEAM_CORE)
+      return v == 0   ? hf(io.rho, lon, lat, k, 0, c.b)
+             : v == 1 ? hf(io.temperature, lon, lat, k, 0, c.b)
+                      : hf(io.velocity, lon, lat, k, v - 2, c.b);
+    const gitm_vert_field &g = KIND == TEAM_DENSITY ? io.ndensity_s
+                               : KIND == TEAM_WIND  ? io.vertical_velocity
+                                                    : io.idensity_s;
+    return hf(g, lon, lat, k, s0 + v, c.b);
+  };
+  double below[N];  // own cell at the level below, as the step leaves it
+#pragma unroll
+  for (int v = 0; v < N; v++) below[v] = *at(v, c.i, c.jl, 0);
+#pragma unroll 1
+  for (int k = 1; k <= p.n_alts; k++) {
+    c.k = k;
+    for (int r2 = cell; r2 < plane; r2 += team_threads) {
+      const int lat = r2 / NLo - 1, lon = r2 % NLo - 1;
+#pragma unroll
+      for (int v = 0; v < N; v++) mine[v * plane + r2] = *at(v, lon, lat, k);
+    }
+    double g[6], ive = 0.0, ivn = 0.0;
+    hz_geometry<true>(c, io, f, nlo, nla);
+    if (KIND == TEAM_CORE) hz_cell_inputs(c, io, f, g);
+    if (KIND == TEAM_ION) {
+      ive = *hf(io.ivelocity, c.i, c.jl, k, 0, c.b);
+      ivn = *hf(io.ivelocity, c.i, c.jl, k, 1, c.b);
+    }
+    double dz[N], orig[N], acc[N], u[N];
+#pragma unroll
+    for (int v = 0; v < N; v++) {
+      dz[v] = c.hz * (*at(v, c.i, c.jl, k + 1) - below[v]);
+      GV_HERE(dz[v]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int v = 0; v < N; v++) orig[v] = x[v * plane];
+#pragma unroll 1
+    for (int stage = 0; stage < 4; stage++) {
+      double go[N], ga[N], d[N];
+      if (active) {
+#pragma unroll
+        for (int v = 0; v < N; v++)
+          hz_gd<true>(c, x + v * plane, NLo, p.beta, dz[v], go[v], ga[v], d[v]);
+        if (KIND == TEAM_CORE) {
+          const double vn = x[(V_VEL + 1) * plane];
+          pub[cell] = x[V_VEL * plane];
+          pub[cells + cell] = vn;
+          pub[2 * cells + cell] = ga[V_VEL + 1] + go[V_VEL] - g[3] * vn * g[0];
+        }
+      }
+      __syncthreads();
+      if (active) {
+        const double ve = KIND == TEAM_ION ? ive : pub[cell],
+                     vn = KIND == TEAM_ION ? ivn : pub[cells + cell], div = pub[2 * cells + cell];
+        if constexpr (KIND == TEAM_CORE) {
+          hz_core_update(p, g, x[V_RHO * plane], x[V_TEMP * plane], ve, vn,
+                         x[(V_VEL + 2) * plane], div, go, ga, d, u);
+        } else {
+#pragma unroll
+          for (int v = 0; v < N; v++)
+            u[v] = hz_carried_update<KIND - 1>(x[v * plane], p.dt, go[v], ga[v], d[v], ve, vn, div);
+        }
+#pragma unroll
+        for (int v = 0; v < N; v++) {
+          u[v] = hz_rk(stage, u[v], x[v * plane], orig[v], acc[v]);
+          // the slices are a team's own, and its lanes have read the stage's
+          // state before the barrier
+          x[v * plane] = u[v];
+        }
+      }
+      __syncthreads();
+    }
+    if (active) {
+      if constexpr (KIND == TEAM_CORE) {
+        hz_store_core(c, io, f, u, orig[V_TEMP]);
+      } else if (KIND == TEAM_ION) {
+#pragma unroll
+        for (int v = 0; v < N; v++) u[v] = hz_store_ion(c, io, v, u[v]);
+        hz_store_electrons(c, io);
+      } else {
+        bool negative = false;
+#pragma unroll
+        for (int v = 0; v < N; v++) {
+          negative = negative || u[v] < 0.0;
+          *at(v, c.i, c.jl, k) = u[v];
+        }
+        if (KIND == TEAM_DENSITY && negative) hz_report(c, nlo, nla, err);
+      }
+    }
+#pragma unroll
+    for (int v = 0; v < N; v++) below[v] = u[v];
   }
+}
+
+// (VP 3: blocks of up to 128 cells, six teams of two wavefronts; VP 6: up to
+// 256 cells, four teams)
+template <bool IONS, int VP, int BLON, int BLAT>
+__global__ void __launch_bounds__(VP == 3 ? 768 : 1024)
+    horiz_topo_kernel(HzParams p, gitm_vert_columns io, HzFields f, unsigned long long *err,
+                      int team_threads) {
+  extern __shared__ double lds[];
+  const int nlo = BLON ? BLON : p.n_lons, nla = BLAT ? BLAT : p.n_lats;
+  const int plane = (nla + 4) * (nlo + 4);
+  const int team = __builtin_amdgcn_readfirstlane((int)threadIdx.x / team_threads);
+  const int cell = (int)threadIdx.x - team * team_threads;
+  double *const slices = lds + hz_pad(nlo);
+  // ve, vn and div of each cell
+  double *const pub = slices + (IONS ? NV_IONS : NV_NEUTRAL) * plane + hz_pad(nlo);
+  constexpr int T = gv::NSP / VP;  // teams per species field
+  if (team == 0)
+    topo_team<TEAM_CORE, NCORE, BLON, BLAT>(p, io, f, err, slices, pub, cell, team_threads, 0);
+  else if (team <= T)
+    topo_team<TEAM_DENSITY, VP, BLON, BLAT>(p, io, f, err, slices, pub, cell, team_threads,
+                                            (team - 1) * VP);
+  else if (team <= 2 * T)
+    topo_team<TEAM_WIND, VP, BLON, BLAT>(p, io, f, err, slices, pub, cell, team_threads,
+                                         (team - 1 - T) * VP);
+  else if (IONS)
+    topo_team<TEAM_ION, NIA, BLON, BLAT>(p, io, f, err, slices, pub, cell, team_threads, 0);
 }
 
 // UseImprovedIonAdvection (advance_horizontal.f90:432-518), after the
@@ -588,20 +847,24 @@ extern "C" int gitm_horiz_advance(gitm_vert_handle *h, const gitm_horiz_params *
     for (const gitm_vert_field *g : {&dv.ivel_par, &dv.glm, &dv.gl0, &dv.glp, &dv.gam, &dv.ga0,
                                      &dv.gap})
       if (!g->ptr) return GITM_VERT_EINVAL;
-  const int nv = ions ? NV_IONS : NV_NEUTRAL;
-  // per altitude: the slab of every variable with halo cells, then the
-  // stage's new values of the block's cells
-  const size_t slab = (size_t)nv * ((nla + 4) * (nlo + 4) + cells) * sizeof(double);
-  // altitudes per workgroup: as many as fit 256 lanes and 40 KB of LDS, so
-  // that four workgroups share a CU (two wavefronts per SIMD, the register
-  // limit); 9x9 blocks take one
-  // (with topography one altitude per workgroup, whatever is asked)
-  int apw = topo ? 1 : hp->altitudes_per_workgroup > 0 ? hp->altitudes_per_workgroup : 0;
-  if (apw == 0) {
-    apw = 1;
-    while ((apw + 1) * cells <= 256 && (apw + 1) * slab <= 40 * 1024 && apw < 4) apw++;
+  const int nv = ions ? NV_IONS : NV_NEUTRAL, plane = (nla + 4) * (nlo + 4);
+  // altitudes per workgroup: what the caller asks (at most 256 lanes, and the
+  // slab of every variable with its new values in a CU's LDS), else as many as
+  // fill 256 lanes with 40 KB of LDS, but no more than leave two workgroups
+  // per CU; with topography a workgroup takes a block, whatever is asked
+  const size_t slab = (size_t)nv * (plane + cells) * sizeof(double);
+  int apw = 1;
+  if (topo) {
+    if (slab > 160 * 1024) return GITM_VERT_EINVAL;
+  } else if (hp->altitudes_per_workgroup > 0) {
+    apw = hp->altitudes_per_workgroup;
+    if (apw * cells > 256 || apw * slab > 160 * 1024) return GITM_VERT_EINVAL;
+  } else {
+    if (slab > 160 * 1024) return GITM_VERT_EINVAL;
+    const size_t group = (size_t)HZ_GROUP * plane * sizeof(double);
+    const long long most = (long long)c->n_alts * c->n_blocks / 512;
+    while ((apw + 1) * cells <= 256 && (apw + 1) * group <= 40 * 1024 && apw + 1 <= most) apw++;
   }
-  if (apw * cells > 256 || apw * slab > 160 * 1024) return GITM_VERT_EINVAL;
   apw = std::min(apw, c->n_alts);
   HzParams p;
   p.dt = hp->dt;
@@ -614,7 +877,6 @@ extern "C" int gitm_horiz_advance(gitm_vert_handle *h, const gitm_horiz_params *
   p.n_blocks = c->n_blocks;
   p.apw = apw;
   p.alt_groups = topo ? 1 : (c->n_alts + apw - 1) / apw;
-  p.k_first = 1;
   const long long nwg = (long long)p.alt_groups * c->n_blocks;
   if (nwg > 0x7fffffffLL) return GITM_VERT_EINVAL;
   HzFields f;
@@ -633,68 +895,37 @@ extern "C" int gitm_horiz_advance(gitm_vert_handle *h, const gitm_horiz_params *
   f.dalt_dlon = hf_->dalt_dlon;
   f.dalt_dlat = hf_->dalt_dlat;
   GV_HIP(hipSetDevice(h->device));
-  const int threads = ((apw * cells + 63) / 64) * 64;
-  const size_t lds = (size_t)apw * slab;
-  // the RK4 sums, in the handle's scratch (shared with the vertical step's
-  // carries: both only use it within a launch on the handle's stream)
-  const size_t need = (size_t)nwg * apw * nv * cells * sizeof(double);
-  if (h->scratch_bytes < need) {
-    if (h->scratch) {
-      GV_HIP(hipStreamSynchronize(h->stream));
-      (void)hipFree(h->scratch);
-      h->scratch = nullptr;
-      h->scratch_bytes = 0;
-    }
-    if (hipMalloc(&h->scratch, need) != hipSuccess) return GITM_VERT_ENOMEM;
-    h->scratch_bytes = need;
-  }
   // GITM's default 9 x 9 blocks take the kernels with the block shape fixed
   const bool b99 = nlo == 9 && nla == 9;
-  auto launch = [&](const HzParams &q) -> int {
-    const dim3 grid((unsigned)nwg), block(threads);
-    if (ions && topo) {
-      if (b99)
-        hipLaunchKernelGGL((horiz_kernel<NV_IONS, true, 9, 9>), grid, block, lds, h->stream, q,
-                           *c, f, h->d_err, h->scratch);
-      else
-        hipLaunchKernelGGL((horiz_kernel<NV_IONS, true>), grid, block, lds, h->stream, q, *c,
-                           f, h->d_err, h->scratch);
-    } else if (ions) {
-      if (b99)
-        hipLaunchKernelGGL((horiz_kernel<NV_IONS, false, 9, 9>), grid, block, lds, h->stream,
-                           q, *c, f, h->d_err, h->scratch);
-      else
-        hipLaunchKernelGGL((horiz_kernel<NV_IONS, false>), grid, block, lds, h->stream, q, *c,
-                           f, h->d_err, h->scratch);
-    } else if (topo) {
-      if (b99)
-        hipLaunchKernelGGL((horiz_kernel<NV_NEUTRAL, true, 9, 9>), grid, block, lds,
-                           h->stream, q, *c, f, h->d_err, h->scratch);
-      else
-        hipLaunchKernelGGL((horiz_kernel<NV_NEUTRAL, true>), grid, block, lds, h->stream, q,
-                           *c, f, h->d_err, h->scratch);
-    } else {
-      if (b99)
-        hipLaunchKernelGGL((horiz_kernel<NV_NEUTRAL, false, 9, 9>), grid, block, lds,
-                           h->stream, q, *c, f, h->d_err, h->scratch);
-      else
-        hipLaunchKernelGGL((horiz_kernel<NV_NEUTRAL, false>), grid, block, lds, h->stream, q,
-                           *c, f, h->d_err, h->scratch);
-    }
-    GV_HIP(hipGetLastError());
-    return GITM_VERT_OK;
-  };
+  const int lanes = ((apw * cells + 63) / 64) * 64;
+  const dim3 grid((unsigned)nwg);
   if (topo) {
-    // one launch per altitude, in order on the stream (:150-430)
-    for (int k = 1; k <= c->n_alts; k++) {
-      p.k_first = k;
-      const int rc = launch(p);
-      if (rc) return rc;
-    }
+    // teams of three variables where six of them fit a workgroup, else of six
+    const bool three = lanes <= 128;
+    const dim3 block((1 + (three ? 4 : 2) + (ions ? 1 : 0)) * lanes);
+    const size_t lds =
+        ((size_t)nv * plane + 2 * hz_pad(nlo) + 3 * (size_t)cells) * sizeof(double);
+    const auto launch = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, grid, block, lds, h->stream, p, *c, f, h->d_err, lanes);
+    };
+    if (three && b99)
+      ions ? launch(horiz_topo_kernel<true, 3, 9, 9>) : launch(horiz_topo_kernel<false, 3, 9, 9>);
+    else if (three)
+      ions ? launch(horiz_topo_kernel<true, 3, 0, 0>) : launch(horiz_topo_kernel<false, 3, 0, 0>);
+    else
+      ions ? launch(horiz_topo_kernel<true, 6, 0, 0>) : launch(horiz_topo_kernel<false, 6, 0, 0>);
   } else {
-    const int rc = launch(p);
-    if (rc) return rc;
+    const size_t lds =
+        ((size_t)apw * HZ_GROUP * plane + 2 * hz_pad(nlo)) * sizeof(double);
+    const auto launch = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, grid, dim3(lanes), lds, h->stream, p, *c, f, h->d_err);
+    };
+    if (b99)
+      ions ? launch(horiz_flat_kernel<true, 9, 9>) : launch(horiz_flat_kernel<false, 9, 9>);
+    else
+      ions ? launch(horiz_flat_kernel<true, 0, 0>) : launch(horiz_flat_kernel<false, 0, 0>);
   }
+  GV_HIP(hipGetLastError());
   if (improved) {
     const long long n =
         (long long)(nlo + 4) * (nla + 4) * (c->n_alts + 4) * (long long)c->n_blocks;

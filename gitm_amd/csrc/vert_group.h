@@ -31,20 +31,6 @@
 
 #include "vert_column.h"
 
-// Keeps the instruction scheduler from interleaving what stands before and
-// after: left alone it overlaps a dozen exponentials for parallelism that the
-// other wavefronts give anyway, and spills what that holds live.
-// GV_HERE(x) makes x be formed where it is written: a value that is used much
-// later is otherwise formed there, and what it is made of (a dozen LDS loads)
-// stays in registers across the phases between.
-#ifdef GV_HOST_EMULATION
-#define GV_ORDER()
-#define GV_HERE(x)
-#else
-#define GV_ORDER() __builtin_amdgcn_sched_barrier(0)
-#define GV_HERE(x) asm volatile("" : "+v"(x))
-#endif
-
 namespace gv {
 
 constexpr int SPW = 2;         // species per lane

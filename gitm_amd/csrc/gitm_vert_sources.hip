@@ -5,16 +5,31 @@
 // (calc_conduction.f90:132-244) and the second-order combination
 // (2H - F) - Q, then the updates of add_sources.f90:53-70,94-107.
 //
-// Mapping: one workgroup per column, one lane per level (blockDim =
-// nAlts+4), as the vertical step.  The tridiagonal (Thomas) solves are
-// serial in altitude, so everything that is not is taken out of them: the
-// lanes stage the column one level each (coalesced loads), form every
-// solve's coefficients one level each, and the serial lanes (one per solve
-// and quantity: 0 the temperature, 1-2 the east and north winds, 3-8 the
-// species' vertical winds) run only the recurrences.  The two Dt/2 solves
-// have the same matrix, so the second reuses the first's pivots and cp and
-// runs only its dp recurrence.  Operations keep the reference's order: the
-// results equal the oracle's bit for bit.
+// Mapping: one workgroup per column, one lane per level, as the vertical
+// step's.  The tridiagonal (Thomas) solves are serial in altitude and the
+// results are the oracle's bit for bit, so neither a parallel solver nor a
+// multiplication by a rounded reciprocal will do; what is left is to make
+// the serial part short and to keep enough columns on a CU to hide it:
+//  * the quotients are the hardware's own division sequence without its
+//    scaling and special cases (div_neg), whose reciprocal a pivot's two
+//    quotients share; range tests beside the chains tell whether that was
+//    exact, and a column where it may not have been is done again with plain
+//    divisions;
+//  * a chain reads ahead, two levels per LDS access (rows of the LDS image
+//    run along altitude), and holds little but its arithmetic: per level the
+//    first sweeps take 150 clocks, of which 88 are the serial operations, the
+//    back substitutions 42;
+//  * the second Dt/2 solve finds the pivots and their reciprocals formed by
+//    the level lanes, so a level of its sweep is five dependent operations,
+//    70 clocks;
+//  * the LDS image is 45 doubles per level (five rows per quantity, each
+//    reused as soon as it is read), four columns of 100 levels per CU.
+// What bounds it is the serial chains of the few columns that the LDS holds:
+// 34 of a column's 65 thousand clocks (LDS writes of 26 clocks each on top of
+// the arithmetic), with 1.6 TB/s of HBM in use.  64,800 columns of 100 levels
+// took 3.25 ms with a division in each link of the chains, 63 doubles per
+// level and no read ahead; they take 1.72 ms.  A column done again costs what
+// it cost then: the plain pass has no read ahead, but four columns per CU.
 #include "vert_gpu.h"
 
 namespace {
@@ -31,39 +46,129 @@ struct SrcFields {
       user_heating, conduction, viscosity, vvisc;
 };
 
+struct SrcArgs {
+  SrcParams p;
+  gitm_vert_columns io;
+  SrcFields f;
+};
+
 constexpr int NQ = 3 + gv::NSP;  // temperature, two winds, six species winds
 
-// LDS record of one level (doubles), per quantity q:
-//   R_A, R_C   the tridiagonal a and c, shared by the three solves (they do
-//              not depend on the step); at the top level, where a does,
-//              R_C holds the Dt solve's a (c is 0 there);
-//   R_BA       b of the Dt/2 solves, then the pivots b - cp a, which the
-//              two Dt/2 solves share (same a, b and c, so the same cp);
-//   R_BC       b of the Dt solve, then its cp; then the second Dt/2
-//              solve's right side, its dp and its solution;
-//   R_DA, R_DC d of the first Dt/2 solve and of the Dt solve, then their
-//              dp, then their solutions;
-//   R_CPA      the Dt/2 solves' cp.  Until the coefficients are formed this
-//              region holds the diffusion coefficients times r^2 (one slot
-//              for the two winds, whose coefficients are equal) and the
-//              altitude.
+// Rows of the LDS image, one per quantity q (RS doubles each, level k at
+// k + 1):
+//   W_A   the tridiagonal a, shared by the three solves (it does not depend
+//         on the step, but at the top level);
+//   W_C   c, read by both solves, then the Dt solve's dp and its solution;
+//         at the top level, where c is 0, the Dt solve's a; then the second
+//         Dt/2 solve's right side, its dp and its solution;
+//   W_BA  b of the Dt/2 solves, then their cp;
+//   W_BC  b of the Dt solve, then its cp; then the reciprocals of the Dt/2
+//         solves' pivots;
+//   W_D   d of the Dt solve (the Dt/2 solve's is twice that in the
+//         interior), then the first Dt/2 solve's dp and its solution; then
+//         the Dt/2 solves' pivots.
+// The two solves' lanes share a wavefront, so both have read c and d of a
+// level before either writes over them.  Until the coefficients are formed
+// the first rows hold the diffusion coefficients times r^2 (one for the two
+// winds, whose coefficients are equal) and the altitude.
 enum {
-  R_A = 0, R_C = R_A + NQ, R_BA = R_C + NQ, R_BC = R_BA + NQ, R_DA = R_BC + NQ,
-  R_DC = R_DA + NQ, R_CPA = R_DC + NQ, R_LEN = R_CPA + NQ,
-  R_DI = R_CPA, R_ALT = R_CPA + NQ - 1
+  W_A = 0, W_C = W_A + NQ, W_BA = W_C + NQ, W_BC = W_BA + NQ, W_D = W_BC + NQ, W_LEN = W_D + NQ,
+  W_DI = 0, W_ALT = NQ - 1
 };
-static_assert(R_LEN % 2 == 1, "odd record length: 64-bit LDS accesses stay conflict-free");
+constexpr int ND = NQ - 1;  // distinct diffusion coefficients
 constexpr int di_slot(int q) { return q == 0 ? 0 : (q < 3 ? 1 : q - 1); }
-static_assert(di_slot(NQ - 1) < NQ - 1, "diffusion slots below the altitude's");
+static_assert(di_slot(NQ - 1) == ND - 1 && W_ALT >= ND, "diffusion rows below the altitude's");
+static_assert(2 * NQ <= 64, "both solves' lanes in one wavefront");
+
+// Doubles of a row: even, so that level 1 and every second one after it are
+// 16-byte aligned, and odd in pairs, so that the chain lanes' rows fall on
+// different LDS banks.
+constexpr int row_len(int n_alts) { return (n_alts + 4) + ((2 - (n_alts + 4)) & 3); }
+
+// IEEE division without its range handling.  The hardware's sequence is:
+// scale both operands, refine v_rcp_f64 twice, multiply, correct by the
+// remainder, undo the scaling and fix special operands up.  The scalings are
+// by powers of two, so where neither the operands nor the remainder leave the
+// normal range the middle part alone gives the same bits: div_recip's refined
+// reciprocal, which quotients by one divisor share, and a multiplication and
+// correction.  div_pos is for divisors > 0 and div_neg for divisors < 0: they
+// differ in the sign of a zero remainder, which makes the quotients of +0 and
+// -0 right too.
+__device__ __forceinline__ double div_recip(double d) {
+  double r = __builtin_amdgcn_rcp(d);
+  r = __builtin_fma(__builtin_fma(-d, r, 1.0), r, r);
+  return __builtin_fma(__builtin_fma(-d, r, 1.0), r, r);
+}
+__device__ __forceinline__ double div_pos(double n, double d, double r) {
+  const double q = n * r;
+  return __builtin_fma(-__builtin_fma(d, q, -n), r, q);
+}
+__device__ __forceinline__ double div_neg(double n, double d, double r) {
+  const double q = n * r;
+  return __builtin_fma(__builtin_fma(-d, q, n), r, q);
+}
+
+// Whether the quick divisions may be used is decided by range.  Divisors
+// known before the chains are positive and within 2^-200..2^200, numerators
+// zero or within 2^-200..2^200, matrix elements within 2^200; the pivots are
+// negative and within 2^-256..2^256 (Pivots), the forward sweeps' values
+// zero throughout or above 2^-600 throughout, and what comes out finite.
+// Otherwise the column is done again with plain divisions.
+struct Range {
+  double lo = 0x1p200, hi = 0.0;  // of the divisors, and of every magnitude
+  bool tiny = false;
+  __device__ __forceinline__ void divisor(double x) {
+    lo = fmin(lo, x);
+    hi = fmax(hi, x);
+  }
+  __device__ __forceinline__ void element(double x) { hi = fmax(hi, fabs(x)); }
+  __device__ __forceinline__ void numerator(double x) {
+    element(x);
+    tiny |= (x != 0.0) & (fabs(x) < 0x1p-200);
+  }
+  __device__ bool good() const { return (lo > 0x1p-200) & (hi < 0x1p200) & !tiny; }
+};
+
+// The ranges of a chain's pivots and values, from the high words of two
+// levels at once (as integers negative doubles ascend with their magnitude;
+// as floats the words' magnitudes compare as the doubles').
+struct Pivots {
+  int lo = 0x7fffffff, hi = (int)0x80000000;
+  __device__ __forceinline__ void see(double x, double y) {
+    lo = min(min(__double2hiint(x), __double2hiint(y)), lo);
+    hi = max(max(__double2hiint(x), __double2hiint(y)), hi);
+  }
+  __device__ bool good() const {
+    return lo >= __double2hiint(-0x1p-256) && hi < __double2hiint(-0x1p256);
+  }
+};
+struct Values {
+  float lo = __builtin_huge_valf(), hi = 0.0f;
+  __device__ __forceinline__ void see(double x, double y) {
+    const float u = __int_as_float(__double2hiint(x)), v = __int_as_float(__double2hiint(y));
+    asm("v_min3_f32 %0, %0, |%1|, |%2|" : "+v"(lo) : "v"(u), "v"(v));
+    asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(hi) : "v"(u), "v"(v));
+  }
+  __device__ bool good() const {
+    return hi == 0.0f || lo >= __int_as_float(__double2hiint(0x1p-600));
+  }
+};
 
 struct SrcCol {
-  const SrcParams &p;
-  const gitm_vert_columns &io;
-  const SrcFields &f;
+  const SrcArgs *args;
   double *lds;
   int ci, cj, cb;
+  int rs;
 
-  __device__ double &rec(int k, int a) const { return lds[(long long)(k + 1) * R_LEN + a]; }
+  // A later phase's view of the arguments: field descriptors and the column's
+  // offsets in them are otherwise read and formed at the kernel's start, and
+  // what the scalar registers do not hold of them is spilled.
+  __device__ __forceinline__ void locate() {
+    asm volatile("" : "+s"(args), "+s"(ci), "+s"(cj), "+s"(cb));
+  }
+
+  __device__ double *row(int w) const { return lds + w * rs + 1; }  // level 0
+  __device__ double &rec(int k, int w) const { return row(w)[k]; }
   __device__ double at(const gitm_vert_field &g, int k, int comp = 0) const {
     return *gv::fld(g, gv::col_base(g, ci, cj, cb), k, comp);
   }
@@ -71,213 +176,535 @@ struct SrcCol {
     return gv::fld(g, gv::col_base(g, ci, cj, cb), k, comp);
   }
   __device__ double quantity(int q, int k) const {
+    const gitm_vert_columns &io = args->io;
     if (q == 0) return at(io.temperature, k);
     if (q < 3) return at(io.velocity, k, q - 1);
     return at(io.vertical_velocity, k, q - 3);
   }
 };
 
+// One quantity's coefficients at one level (calc_conduction.f90:181-230).
+struct Coef {
+  double a, c, ba, bc, d, ma;
+};
+// The grid factors that a level's quantities share.
+struct Grid {
+  double r, du12, du22, r12, r22;
+};
+template <bool FAST>
+__device__ __forceinline__ Coef coefficients(Range &range, int k, int nA, double dtA, double dtC,
+                                             const Grid &g, double told, double mr, double di0,
+                                             double dl) {
+  const auto div = [](double n, double d, double r) { return FAST ? div_pos(n, d, r) : n / d; };
+  const double r = g.r;
+  // Dt is twice Dt/2 without rounding, so the fast form has the Dt solve's
+  // quotients from the Dt/2 solve's
+  const double mA = div(dtA, mr, FAST ? div_recip(mr) : 0.0);
+  const double mC = FAST ? 2.0 * mA : dtC / mr;
+  const double rm = FAST ? div_recip(mA) : 0.0;
+  const bool top = k > nA;
+  const double h = r * (1.0 + r) * di0;
+  const double xn = top ? h * mA : di0;
+  const double x = div(xn, g.du22, g.r22), y = div(dl, g.du12, g.r12);
+  const double i = div(1.0, mA, rm);
+  Coef o;
+  o.ma = mA;
+  o.a = x * r - y * r * r;
+  o.c = x + y;
+  o.ba = -i - x * (1 + r) - y * (1 - r * r);
+  o.bc = (FAST ? -0.5 * i : -1 / mC) - x * (1 + r) - y * (1 - r * r);
+  o.d = FAST ? -0.5 * div(told, mA, rm) : -told / mC;
+  if (FAST) {
+    range.divisor(mr);
+    range.divisor(mA);
+    range.numerator(xn);
+    range.numerator(dl);
+    range.numerator(told);
+    range.numerator(o.c);
+    range.element(o.a);
+    range.element(o.ba);
+    range.element(o.bc);
+  }
+  if (k < 1) {  // a = 0, b = -1, c = 0, d = -told (:210-213)
+    o.a = o.c = 0.0;
+    o.ba = o.bc = -1.0;
+  }
+  if (top) {  // Neumann, :221-230
+    o.a = x;
+    o.c = FAST ? 2.0 * x : h * mC / g.du22;
+    o.ba = -1.0 * (1.0 + o.a);
+    o.bc = -1.0 * (1.0 + o.c);
+  }
+  if (k < 1 || top) o.d = -told;
+  return o;
+}
+
+// Two levels of a row from level i on, i odd: 16-byte aligned.
+__device__ __forceinline__ double2 load2(const double *row, int i) {
+  return *reinterpret_cast<const double2 *>(row + i);
+}
+__device__ __forceinline__ void store2(double *row, int i, double2 v) {
+  *reinterpret_cast<double2 *>(row + i) = v;
+}
+
+// The chains take two levels at a time.  A lone wavefront issues one
+// instruction of whatever kind every 4 to 5 clocks and an LDS read takes some
+// 60, so the loops hold nothing but arithmetic, 16-byte LDS accesses and an
+// address per row: a ring of P pairs holds operands on their way, a pair's
+// slot is read anew as soon as its levels are done, U rounds of the ring are
+// unrolled, and what is read past the last pair (within the LDS image, PAD
+// doubles beyond its last row) is not used.  step(slot, i) works on levels i
+// and i + 1 and read(slot, i) starts its reads; n pairs from level i0 on in
+// steps of d levels.
+template <int P, int U, class Slot, class Read, class Step>
+__device__ __forceinline__ void ring(int n, int i0, int d, const Read &read, const Step &step) {
+  Slot x[P];
+#pragma unroll
+  for (int p = 0; p < P; p++) read(x[p], i0 + p * d);
+  int i = i0;
+  for (; n >= P * U; n -= P * U, i += P * U * d) {
+#pragma unroll
+    for (int p = 0; p < P * U; p++) {
+      step(x[p % P], i + p * d);
+      GV_ORDER();
+      read(x[p % P], i + (p + P) * d);
+      GV_ORDER();
+    }
+  }
+#pragma unroll
+  for (int p = 0; p < P * U - 1; p++)
+    if (p < n) {
+      step(x[p % P], i + p * d);
+      if (p + P < P * U - 1) read(x[p % P], i + (p + P) * d);
+    }
+}
+constexpr int PAD = 16;  // ring reads at most P pairs past the last level
+
+// The forward sweep of one solve (:232-241): cp to rb, dp to wd.  sc d is the
+// solve's right side (sc is 1 or 2: the fma rounds once).
+struct Fwd {
+  double2 a, c, b, d;
+};
+// cp at one level, and dp at the level below, whose pivot is known by then:
+// dp's five operations go between those of the pivot's reciprocal, each of
+// which waits 6 to 22 clocks for the one before (88 a level).
+struct Forward {
+  double sc, cp, dp;
+  double a, d, den, r;  // the level below's
+  __device__ __forceinline__ void level(double a1, double c1, double b1, double d1) {
+    const double t = cp * a1;
+    GV_ORDER();
+    const double den1 = b1 - t;
+    const double u = dp * a;
+    GV_ORDER();
+    const double r0 = __builtin_amdgcn_rcp(den1);
+    const double n = __builtin_fma(d, sc, -u);
+    GV_ORDER();
+    const double q = n * r;
+    const double e0 = __builtin_fma(-den1, r0, 1.0);
+    GV_ORDER();
+    const double m = __builtin_fma(-den, q, n);
+    const double r1 = __builtin_fma(e0, r0, r0);
+    GV_ORDER();
+    dp = __builtin_fma(m, r, q);
+    const double e1 = __builtin_fma(-den1, r1, 1.0);
+    GV_ORDER();
+    const double r2 = __builtin_fma(e1, r1, r1);
+    const double qc = c1 * r2;
+    const double mc = __builtin_fma(-den1, qc, c1);
+    cp = __builtin_fma(mc, r2, qc);
+    a = a1;
+    d = d1;
+    den = den1;
+    r = r2;
+  }
+  __device__ __forceinline__ double last() {
+    const double n = __builtin_fma(d, sc, -(dp * a));
+    return dp = div_neg(n, den, r);
+  }
+};
+template <bool FAST>
+__device__ __forceinline__ bool sweep(const double *ra, const double *rc, double *rb,
+                                      const double *rd, double *wd, double sc, int nA, double &cp,
+                                      double &dp) {
+  const auto plain = [&](double a, double c, double b, double d) {
+    const double den = b - cp * a;
+    const double n = __builtin_fma(d, sc, -(dp * a));
+    cp = c / den;
+    dp = n / den;
+    return den;
+  };
+  if (!FAST) {
+    for (int i = 1; i <= nA; i++) {
+      plain(ra[i], rc[i], rb[i], rd[i]);
+      rb[i] = cp;
+      wd[i] = dp;
+    }
+    return true;
+  }
+  Pivots pivots;
+  Values values;
+  // the odd level out, if there is one, is read before the ring runs
+  const double a1 = ra[nA], c1 = rc[nA], b1 = rb[nA], d1 = rd[nA];
+  // the level below level 1 gives dp = dp(0)
+  Forward f{sc, cp, 0.0, 0.0, -dp / sc, -1.0, -1.0};
+  double v0 = dp;
+  ring<2, 4, Fwd>(
+      nA / 2, 1, 2,
+      [&](Fwd &x, int i) {
+        x.b = load2(rb, i);
+        x.a = load2(ra, i);
+        x.c = load2(rc, i);
+        x.d = load2(rd, i);
+      },
+      [&](Fwd &x, int i) {
+        double2 c;
+        f.level(x.a.x, x.c.x, x.b.x, x.d.x);
+        const double p0 = f.den;
+        c.x = f.cp;
+        const double v1 = f.dp;
+        f.level(x.a.y, x.c.y, x.b.y, x.d.y);
+        c.y = f.cp;
+        store2(rb, i, c);
+        store2(wd, i - 2, make_double2(v0, v1));
+        pivots.see(p0, f.den);
+        values.see(v0, v1);
+        v0 = f.dp;
+      });
+  const int top = nA & ~1;
+  cp = f.cp;
+  dp = f.last();
+  values.see(v0, dp);
+  store2(wd, top - 1, make_double2(v0, dp));
+  if (nA & 1) {
+    const double p = plain(a1, c1, b1, d1);
+    pivots.see(p, p);
+    values.see(dp, dp);
+    rb[nA] = cp;
+    wd[nA] = dp;
+  }
+  return pivots.good() && values.good();
+}
+
+// The forward sweep on known pivots: dp over the right side in rn.
+struct Fwd2 {
+  double2 a, n, den, r;
+};
+template <bool FAST>
+__device__ __forceinline__ bool sweep2(const double *ra, double *rn, const double *rden,
+                                       const double *rr, int nA, double &dp) {
+  if (!FAST) {
+    for (int i = 1; i <= nA; i++) rn[i] = dp = (rn[i] - dp * ra[i]) / rden[i];
+    return true;
+  }
+  Values values;
+  const double a1 = ra[nA], n1 = rn[nA], den1 = rden[nA];
+  ring<3, 2, Fwd2>(
+      nA / 2, 1, 2,
+      [&](Fwd2 &x, int i) {
+        x.a = load2(ra, i);
+        x.n = load2(rn, i);
+        x.r = load2(rr, i);
+        x.den = load2(rden, i);
+      },
+      [&](Fwd2 &x, int i) {
+        double2 v;
+        v.x = dp = div_neg(x.n.x - dp * x.a.x, x.den.x, x.r.x);
+        v.y = dp = div_neg(x.n.y - dp * x.a.y, x.den.y, x.r.y);
+        values.see(v.x, v.y);
+        store2(rn, i, v);
+      });
+  if (nA & 1) {
+    rn[nA] = dp = (n1 - dp * a1) / den1;
+    values.see(dp, dp);
+  }
+  return values.good();
+}
+
+// The back substitution (:243-247), levels nA..0: the solution over dp in
+// rd; t the value at nA + 1.
+struct Back {
+  double2 cp, dp;
+};
+template <bool FAST>
+__device__ __forceinline__ void back(const double *rc, double *rd, int nA, double t) {
+  if (!FAST) {
+    for (int i = nA; i >= 0; i--) rd[i] = t = rd[i] - rc[i] * t;
+    return;
+  }
+  const double c0 = rc[0], d0 = rd[0], c1 = rc[nA], d1 = rd[nA];
+  if (nA & 1) rd[nA] = t = d1 - c1 * t;
+  const int n = nA / 2;
+  ring<4, 2, Back>(
+      n, 2 * n - 1, -2,
+      [&](Back &x, int i) {
+        x.cp = load2(rc, i);
+        x.dp = load2(rd, i);
+      },
+      [&](Back &x, int i) {
+        double2 v;
+        v.y = t = x.dp.y - x.cp.y * t;
+        v.x = t = x.dp.x - x.cp.x * t;
+        store2(rd, i, v);
+      });
+  rd[0] = d0 - c0 * t;
+}
+
+// A level's values that outlive the solves.
+struct Level {
+  double qin[NQ], s1[NQ], fv[NQ], h[NQ];  // in, first Dt/2 step, Dt step, second Dt/2 step
+  double unit, vup, vu, heat[3];
+};
+
 // Phases of one column (barriers between them):
 //  1. stage: one lane per level -1..nAlts+2 loads its level; the diffusion
 //     coefficients and the altitude go to LDS, the rest stays in registers;
-//  2. coefficients: one lane per level 0..nAlts+1 forms the grid factors
-//     and every solve's a, b, c and d (calc_conduction.f90:181-230);
+//  2. one lane per level 0..nAlts+1 reads its neighbours', forms the grid
+//     factors and, after a barrier, every solve's a, b, c and d;
 //  3. the forward sweeps and back substitutions of the first Dt/2 solve and
-//     the Dt solve, one lane per (solve, quantity), serial in altitude
-//     (:232-247);
-//  4. one lane per level: the first stage's value, the full step's, and
-//     the second Dt/2 solve's right side;
-//  5. the second Dt/2 solve on the first's pivots and cp: only its dp
-//     recurrence and back substitution, one lane per quantity;
-//  6. one lane per level: the combination (2H - F) - Q (:117-121,
-//     calc_viscosity.f90:110-114), the increments and add_sources' updates.
-template <int NT>
-__global__ void __launch_bounds__(NT)
-    sources_kernel(SrcParams p, gitm_vert_columns io, SrcFields f) {
-  extern __shared__ double lds[];
-  const int col = xcd_column((int)blockIdx.x, (int)gridDim.x), j = (int)threadIdx.x, k = j - 1;
-  const int nA = p.n_alts;
-  const int nlb = io.n_lons * io.n_lats;
+//     the Dt solve, one lane per (solve, quantity) of the first wavefront,
+//     serial in altitude (:232-247);
+//  4. one lane per level: the first stage's value, the full step's, and the
+//     second Dt/2 solve's right side, pivots and reciprocals;
+//  5. the second Dt/2 solve, one lane per quantity, and its values.
+// With FAST the phases end early, for the whole workgroup, once a range test
+// fails; returns whether none did.  Each phase has its own word of failed[]:
+// it is written before a barrier and only read after it.
+template <bool FAST>
+__device__ __forceinline__ bool solves(const SrcCol &c, volatile int *failed, int j,
+                                       Level &v) {
+  const SrcParams &p = c.args->p;
+  const gitm_vert_columns &io = c.args->io;
+  const SrcFields &f = c.args->f;
+  const int k = j - 1, nA = p.n_alts;
   const bool lev = k >= 0 && k <= nA + 1;
-  SrcCol c{p, io, f, lds, col % io.n_lons, (col / io.n_lons) % io.n_lats, col / nlb};
   const double dtA = p.dt / 2.0, dtC = p.dt;
-  double qin[NQ], mr[NQ], unit = 1.0;
+  double mr[NQ];
   // 1. stage
-  c.rec(k, R_ALT) = c.at(io.altitude, k);
+  if (FAST && j < 5) failed[j] = 0;
+  if (k <= nA + 2) c.rec(k, W_ALT) = c.at(io.altitude, k);
   if (lev) {
-    unit = c.at(io.temp_unit, k);
-    const double rd = c.at(f.raddist, k);
-    const double r2 = rd * rd;
-    const double rho = c.at(io.rho, k), eddy = c.at(io.eddy, k);
-    {  // calc_conduction.f90:59-73
-      const double cpk = c.at(f.cp, k);
-      const double prandtl = p.use_turbulent_cond ? eddy * rho * cpk : 0.0;
-      c.rec(k, R_DI + di_slot(0)) = (c.at(f.kappa_temp, k) + prandtl) * r2;
-      mr[0] = (rho * cpk) * r2;
+    v.unit = c.at(io.temp_unit, k);
+    const double rd = c.at(f.raddist, k), rho = c.at(io.rho, k), eddy = c.at(io.eddy, k),
+                 cpk = c.at(f.cp, k), kappa = c.at(f.kappa_temp, k), visc = c.at(f.visc_coef, k);
+    double n[gv::NSP], vs[gv::NSP];
+#pragma unroll
+    for (int s = 0; s < gv::NSP; s++) {
+      n[s] = c.at(io.ndensity_s, k, s);
+      vs[s] = c.at(f.visc_coef_s, k, s);
     }
+#pragma unroll
+    for (int q = 0; q < NQ; q++) v.qin[q] = c.quantity(q, k);
+    // what the updates add to, read while nothing waits for it
+    if (p.apply) {
+      v.vu = c.at(io.velocity, k, 2);
+      if (k >= 1 && k <= nA) {
+        if (f.heating.ptr) v.heat[0] = c.at(f.heating, k);
+        if (f.chem_heating.ptr) v.heat[1] = c.at(f.chem_heating, k);
+        if (f.user_heating.ptr) v.heat[2] = c.at(f.user_heating, k);
+      }
+    }
+    GV_ORDER();  // every load is under way before the first is waited for
+    const double r2 = rd * rd;
+    // calc_conduction.f90:59-73
+    const double prandtl = p.use_turbulent_cond ? eddy * rho * cpk : 0.0;
+    c.rec(k, W_DI + di_slot(0)) = (kappa + prandtl) * r2;
+    mr[0] = (rho * cpk) * r2;
     // calc_viscosity.f90:66-67
-    c.rec(k, R_DI + di_slot(1)) = (c.at(f.visc_coef, k) + rho * eddy) * r2;
+    c.rec(k, W_DI + di_slot(1)) = (visc + rho * eddy) * r2;
     mr[1] = rho * r2;
     mr[2] = rho * r2;
 #pragma unroll
     for (int s = 0; s < gv::NSP; s++) {  // :125-128
-      const double n = c.at(io.ndensity_s, k, s);
-      const double mn = p.mass[s] * n;
-      c.rec(k, R_DI + di_slot(3 + s)) =
-          ((4.0 / 3.0) * c.at(f.visc_coef_s, k, s) + mn * eddy) * r2;
-      mr[3 + s] = (p.mass[s] * n) * r2;
+      const double mn = p.mass[s] * n[s];
+      c.rec(k, W_DI + di_slot(3 + s)) = ((4.0 / 3.0) * vs[s] + mn * eddy) * r2;
+      mr[3 + s] = mn * r2;
     }
-#pragma unroll
-    for (int q = 0; q < NQ; q++) qin[q] = c.quantity(q, k);
   }
   __syncthreads();
-  // 2. coefficients; they read only R_CPA's region and write the others
+  // 2. coefficients
+  Grid g;
+  double di[ND], dl[ND], ba[NQ], ma[NQ];
+  Range range;
   if (lev) {
-    const double altm = c.rec(k - 1, R_ALT), alt0 = c.rec(k, R_ALT),
-                 altp = c.rec(k + 1, R_ALT);
+    const double altm = c.rec(k - 1, W_ALT), alt0 = c.rec(k, W_ALT),
+                 altp = c.rec(k + 1, W_ALT);
     const double du = altp - alt0, dl0 = alt0 - altm;  // :181-186
     const double r = du / dl0;
-    const double du12 = du * du * (1 + r) * (1 + r);
-    const double du22 = 0.5 * (dl0 * du + du * du);
+    g.r = r;
+    g.du12 = du * du * (1 + r) * (1 + r);
+    g.du22 = 0.5 * (dl0 * du + du * du);
+    if (FAST) {
+      g.r12 = div_recip(g.du12);
+      g.r22 = div_recip(g.du22);
+      range.divisor(g.du12);
+      range.divisor(g.du22);
+    }
 #pragma unroll
-    for (int q = 0; q < NQ; q++) {
-      const double told = q == 0 ? qin[0] * unit : qin[q];
-      const double di0 = c.rec(k, R_DI + di_slot(q));
-      if (k == 0) {  // a = 0, b = -1, c = 0, d = -told (:210-213)
-        c.rec(k, R_A + q) = 0.0;
-        c.rec(k, R_C + q) = 0.0;
-        c.rec(k, R_BA + q) = -1.0;
-        c.rec(k, R_BC + q) = -1.0;
-        c.rec(k, R_DA + q) = -told;
-        c.rec(k, R_DC + q) = -told;
-      } else if (k <= nA) {
-        const double mA = dtA / mr[q], mC = dtC / mr[q];
-        const double dl = c.rec(k + 1, R_DI + di_slot(q)) -
-                          r * r * c.rec(k - 1, R_DI + di_slot(q)) -
-                          (1 - r * r) * di0;  // :188-190
-        c.rec(k, R_A + q) = di0 / du22 * r - dl / du12 * r * r;
-        c.rec(k, R_C + q) = di0 / du22 + dl / du12;
-        c.rec(k, R_BA + q) = -1 / mA - di0 / du22 * (1 + r) - dl / du12 * (1 - r * r);
-        c.rec(k, R_BC + q) = -1 / mC - di0 / du22 * (1 + r) - dl / du12 * (1 - r * r);
-        c.rec(k, R_DA + q) = -told / mA;
-        c.rec(k, R_DC + q) = -told / mC;
-      } else {  // Neumann top, :221-230
-        const double mA = dtA / mr[q], mC = dtC / mr[q];
-        c.rec(k, R_A + q) = 1.0 * (r * (1.0 + r) * di0 * mA / du22);
-        c.rec(k, R_C + q) = 1.0 * (r * (1.0 + r) * di0 * mC / du22);
-        c.rec(k, R_BA + q) = -1.0 * (1.0 + r * (1 + r) * di0 * mA / du22);
-        c.rec(k, R_BC + q) = -1.0 * (1.0 + r * (1 + r) * di0 * mC / du22);
-        c.rec(k, R_DA + q) = -told;
-        c.rec(k, R_DC + q) = -told;
-      }
-    }
+    for (int s = 0; s < ND; s++) di[s] = dl[s] = c.rec(k, W_DI + s);
+    if (k >= 1 && k <= nA)
+#pragma unroll
+      for (int s = 0; s < ND; s++)
+        dl[s] = c.rec(k + 1, W_DI + s) - r * r * c.rec(k - 1, W_DI + s) -
+                (1 - r * r) * di[s];  // :188-190
   }
   __syncthreads();
-  // 3. the first Dt/2 solve (A) and the Dt solve (C), at once (columns of
-  // fewer than 18 levels take some in turn)
-  for (int task = j; task < 2 * NQ; task += (int)blockDim.x) {
-    const int q = task % NQ;
-    const bool isA = task < NQ;
-    // b's slot takes the pivot, then (for C, where cs == bs) cp
-    const int bs = (isA ? R_BA : R_BC) + q, ds = (isA ? R_DA : R_DC) + q,
-              cs = (isA ? R_CPA : R_BC) + q;
-    double cpv = 0.0 / -1.0;
-    double dpv = c.rec(0, ds) / -1.0;
-    c.rec(0, cs) = cpv;
-    c.rec(0, ds) = dpv;
-    for (int i = 1; i <= nA; i++) {
-      const double a = c.rec(i, R_A + q), cc = c.rec(i, R_C + q);
-      const double den = c.rec(i, bs) - cpv * a;
-      const double cpn = cc / den;
-      const double dpn = (c.rec(i, ds) - dpv * a) / den;
-      c.rec(i, bs) = den;
-      c.rec(i, cs) = cpn;
-      c.rec(i, ds) = dpn;
-      cpv = cpn;
-      dpv = dpn;
-    }
-    const int top = nA + 1;
-    const double a = c.rec(top, (isA ? R_A : R_C) + q);
-    const double den = c.rec(top, bs) - cpv * a;
-    double t = (c.rec(top, ds) - dpv * a) / den;  // temp(nAlts+1) = dp(nAlts+1)
-    c.rec(top, bs) = den;
-    c.rec(top, ds) = t;
-    for (int i = nA; i >= 0; i--) {
-      t = c.rec(i, ds) - c.rec(i, cs) * t;
-      c.rec(i, ds) = t;
-    }
-  }
-  __syncthreads();
-  // 4. the first stage's value s1 and the full step's fv (dTdt_cond,
-  // :249-250), and the second Dt/2 solve's right side
-  double s1[NQ], fv[NQ], vup = 0.0;
   if (lev) {
 #pragma unroll
     for (int q = 0; q < NQ; q++) {
-      const double in = q == 0 ? qin[0] * unit : qin[q];
-      const double ra = c.rec(k, R_DA + q) - in, rc = c.rec(k, R_DC + q) - in;
-      s1[q] = q == 0 ? qin[0] + ra / unit : qin[q] + ra;
-      fv[q] = q == 0 ? qin[0] + rc / unit : qin[q] + rc;
+      const double told = q == 0 ? v.qin[0] * v.unit : v.qin[q];
+      const Coef o = coefficients<FAST>(range, k, nA, dtA, dtC, g, told, mr[q], di[di_slot(q)],
+                                        dl[di_slot(q)]);
+      c.rec(k, W_A + q) = o.a;
+      c.rec(k, W_C + q) = o.c;
+      c.rec(k, W_BA + q) = ba[q] = o.ba;
+      c.rec(k, W_BC + q) = o.bc;
+      c.rec(k, W_D + q) = o.d;
+      ma[q] = o.ma;
+    }
+    if (FAST && !range.good()) failed[0] = 1;
+  }
+  __syncthreads();
+  if (FAST && __builtin_amdgcn_readfirstlane(failed[0])) return false;
+  // 3. the first Dt/2 solve (A) and the Dt solve (C), at once
+  if (j < 2 * NQ) {
+    const bool isA = j < NQ;
+    const int q = isA ? j : j - NQ, top = nA + 1;
+    const double *ra = c.row(W_A + q), *rc = c.row(W_C + q), *rd = c.row(W_D + q);
+    double *rb = c.row((isA ? W_BA : W_BC) + q), *wd = c.row((isA ? W_D : W_C) + q);
+    const double a = (isA ? ra : rc)[top], b = rb[top], d = rd[top];
+    double cp = 0.0 / -1.0;
+    double dp = rd[0] / -1.0;
+    rb[0] = cp;
+    wd[0] = dp;
+    if (!sweep<FAST>(ra, rc, rb, rd, wd, isA ? 2.0 : 1.0, nA, cp, dp)) failed[1] = 1;
+    const double t = (d - dp * a) / (b - cp * a);  // temp(nAlts+1) = dp(nAlts+1)
+    wd[top] = t;
+    back<FAST>(rb, wd, nA, t);
+  }
+  __syncthreads();
+  if (FAST && __builtin_amdgcn_readfirstlane(failed[1])) return false;
+  // 4. the first stage's value s1 and the full step's fv (dTdt_cond,
+  // :249-250), and the second Dt/2 solve's operands
+  if (lev) {
+    double finite = 0.0;
+    Range told_range;
+#pragma unroll
+    for (int q = 0; q < NQ; q++) {
+      const double in = q == 0 ? v.qin[0] * v.unit : v.qin[q];
+      const double ra = c.rec(k, W_D + q) - in, rc = c.rec(k, W_C + q) - in;
+      v.s1[q] = q == 0 ? v.qin[0] + ra / v.unit : v.qin[q] + ra;
+      v.fv[q] = q == 0 ? v.qin[0] + rc / v.unit : v.qin[q] + rc;
       // Viscosity(:,:,:,iUp_) keeps the last species' full-step result
       // (calc_viscosity.f90:161)
-      if (q == NQ - 1) vup = rc;
-      const double told = q == 0 ? s1[0] * unit : s1[q];
-      c.rec(k, R_BC + q) = (k >= 1 && k <= nA) ? -told / (dtA / mr[q]) : -told;
+      if (q == NQ - 1) v.vup = rc;
+      const double told = q == 0 ? v.s1[0] * v.unit : v.s1[q];
+      double rhs;
+      if (FAST) {
+        finite = __builtin_fma(ra, 0.0, __builtin_fma(rc, 0.0, finite));
+        told_range.numerator(told);
+        rhs = -div_pos(told, ma[q], div_recip(ma[q]));
+      } else {
+        rhs = -told / ma[q];
+      }
+      c.rec(k, W_C + q) = k >= 1 && k <= nA ? rhs : -told;
+      if (k >= 1) {
+        const double den = ba[q] - c.rec(k - 1, W_BA + q) * c.rec(k, W_A + q);
+        c.rec(k, W_D + q) = den;
+        if (FAST) c.rec(k, W_BC + q) = div_recip(den);
+      }
     }
+    if (FAST && !(told_range.good() && finite == 0.0)) failed[2] = 1;
   }
   __syncthreads();
-  // 5. the second Dt/2 solve (B): A's pivots and cp, its own dp
-  for (int q = j; q < NQ; q += (int)blockDim.x) {
-    double dpv = c.rec(0, R_BC + q) / -1.0;
-    c.rec(0, R_BC + q) = dpv;
-    for (int i = 1; i <= nA + 1; i++) {
-      dpv = (c.rec(i, R_BC + q) - dpv * c.rec(i, R_A + q)) / c.rec(i, R_BA + q);
-      c.rec(i, R_BC + q) = dpv;
-    }
-    double t = dpv;
-    for (int i = nA; i >= 0; i--) {
-      t = c.rec(i, R_BC + q) - c.rec(i, R_CPA + q) * t;
-      c.rec(i, R_BC + q) = t;
-    }
+  if (FAST && __builtin_amdgcn_readfirstlane(failed[2])) return false;
+  // 5. the second Dt/2 solve (B)
+  if (j < NQ) {
+    const double *ra = c.row(W_A + j), *rden = c.row(W_D + j), *rr = c.row(W_BC + j);
+    double *rn = c.row(W_C + j);
+    const int top = nA + 1;
+    const double a = ra[top], b = rden[top], d = rn[top];
+    double dp = rn[0] / -1.0;
+    rn[0] = dp;
+    if (!sweep2<FAST>(ra, rn, rden, rr, nA, dp)) failed[3] = 1;
+    const double t = (d - dp * a) / b;
+    rn[top] = t;
+    back<FAST>(c.row(W_BA + j), rn, nA, t);
   }
   __syncthreads();
-  if (!lev) return;
-  // 6. the combination, the increments and add_sources' updates
-  // (:53-70, :94-114), one level per lane
+  if (FAST && __builtin_amdgcn_readfirstlane(failed[3])) return false;
+  if (lev) {
+    double finite = 0.0;
+#pragma unroll
+    for (int q = 0; q < NQ; q++) {
+      v.h[q] = c.rec(k, W_C + q);
+      finite = __builtin_fma(v.h[q], 0.0, finite);
+    }
+    if (FAST && !(finite == 0.0)) failed[4] = 1;
+  }
+  if (!FAST) return true;
+  __syncthreads();
+  return __builtin_amdgcn_readfirstlane(failed[4]) == 0;
+}
+
+// Two wavefronts per SIMD are what the LDS image leaves room for: 256 VGPRs.
+template <int NT>
+__global__ void __launch_bounds__(NT, 2)
+    sources_kernel(SrcArgs) {
+  extern __shared__ __align__(16) double lds[];
+  const auto *args = (const SrcArgs *)(const __attribute__((address_space(4))) SrcArgs *)
+      __builtin_amdgcn_kernarg_segment_ptr();
+  const int col = xcd_column((int)blockIdx.x, (int)gridDim.x), j = (int)threadIdx.x, k = j - 1;
+  const int nA = args->p.n_alts, nlon = args->io.n_lons, nlat = args->io.n_lats;
+  SrcCol c{args, lds, col % nlon, (col / nlon) % nlat, col / (nlon * nlat), row_len(nA)};
+  volatile int *failed = reinterpret_cast<volatile int *>(lds + W_LEN * c.rs + PAD);
+  Level v;
+  v.unit = 1.0;
+  v.vu = v.heat[0] = v.heat[1] = v.heat[2] = 0.0;
+  if (!solves<true>(c, failed, j, v)) {
+    __syncthreads();  // every lane is through with LDS
+    c.locate();
+    solves<false>(c, failed, j, v);
+  }
+  c.locate();
+  const SrcParams &p = c.args->p;
+  const gitm_vert_columns &io = c.args->io;
+  const SrcFields &f = c.args->f;
+  if (k < 0 || k > nA + 1) return;
+  // 6. the combination (2H - F) - Q (:117-121, calc_viscosity.f90:110-114),
+  // the increments and add_sources' updates (:53-70, :94-114), one level per
+  // lane
   double out[NQ];
 #pragma unroll
   for (int q = 0; q < NQ; q++) {
-    const double in = q == 0 ? s1[0] * unit : s1[q];
-    const double rb = c.rec(k, R_BC + q) - in;
-    const double h = q == 0 ? s1[0] + rb / unit : s1[q] + rb;
-    out[q] = (2.0 * h - fv[q]) - qin[q];
+    const double in = q == 0 ? v.s1[0] * v.unit : v.s1[q];
+    const double rb = v.h[q] - in;
+    const double h = q == 0 ? v.s1[0] + rb / v.unit : v.s1[q] + rb;
+    out[q] = (2.0 * h - v.fv[q]) - v.qin[q];
   }
   const double cond = out[0];
   if (f.conduction.ptr) *c.ptr(f.conduction, k) = cond;
   if (f.viscosity.ptr) {
     *c.ptr(f.viscosity, k, 0) = out[1];
     *c.ptr(f.viscosity, k, 1) = out[2];
-    *c.ptr(f.viscosity, k, 2) = vup;
+    *c.ptr(f.viscosity, k, 2) = v.vup;
   }
   if (f.vvisc.ptr)
 #pragma unroll
     for (int s = 0; s < gv::NSP; s++) *c.ptr(f.vvisc, k, s) = out[3 + s];
   if (!p.apply) return;
-  double tt = qin[0];
+  double tt = v.qin[0];
   if (k >= 1 && k <= nA) {
-    tt = tt + p.dt * (f.heating.ptr ? c.at(f.heating, k) : 0.0);
-    if (f.chem_heating.ptr) tt = tt + c.at(f.chem_heating, k);
-    if (f.user_heating.ptr) tt = tt + c.at(f.user_heating, k);
+    tt = tt + p.dt * v.heat[0];
+    if (f.chem_heating.ptr) tt = tt + v.heat[1];
+    if (f.user_heating.ptr) tt = tt + v.heat[2];
   }
   *c.ptr(io.temperature, k) = tt + cond;
-  *c.ptr(io.velocity, k, 0) = qin[1] + out[1];
-  *c.ptr(io.velocity, k, 1) = qin[2] + out[2];
-  {
-    double *vu = c.ptr(io.velocity, k, 2);
-    *vu = *vu + vup;
-  }
+  *c.ptr(io.velocity, k, 0) = v.qin[1] + out[1];
+  *c.ptr(io.velocity, k, 1) = v.qin[2] + out[2];
+  *c.ptr(io.velocity, k, 2) = v.vu + v.vup;
 #pragma unroll
-  for (int s = 0; s < gv::NSP; s++) *c.ptr(io.vertical_velocity, k, s) = qin[3 + s] + out[3 + s];
+  for (int s = 0; s < gv::NSP; s++) *c.ptr(io.vertical_velocity, k, s) = v.qin[3 + s] + out[3 + s];
 }
 
 }  // namespace
@@ -300,14 +727,16 @@ extern "C" int gitm_vert_sources(gitm_vert_handle *h, const gitm_vert_sources_pa
   for (int s = 0; s < gv::NSP; s++)
     if (!(sp->mass[s] > 0.0)) return GITM_VERT_EINVAL;
   GV_HIP(hipSetDevice(h->device));
-  SrcParams p;
+  SrcArgs args;
+  SrcParams &p = args.p;
+  args.io = *c;
   p.dt = sp->dt;
   for (int s = 0; s < gv::NSP; s++) p.mass[s] = sp->mass[s];
   p.use_turbulent_cond = sp->use_turbulent_cond != 0;
   p.apply = sp->apply != 0;
   p.n_alts = c->n_alts;
   p.n_cols = (int)ncols;
-  SrcFields f;
+  SrcFields &f = args.f;
   f.kappa_temp = sf->kappa_temp;
   f.visc_coef = sf->visc_coef;
   f.visc_coef_s = sf->visc_coef_s;
@@ -319,14 +748,14 @@ extern "C" int gitm_vert_sources(gitm_vert_handle *h, const gitm_vert_sources_pa
   f.conduction = sf->conduction;
   f.viscosity = sf->viscosity;
   f.vvisc = sf->vertical_viscosity;
-  const size_t lds = (size_t)R_LEN * (size_t)(c->n_alts + 4) * sizeof(double);
-  if (lds > (size_t)160 * 1024) return GITM_VERT_EUNSUPPORTED;  // 129 KB at nAlts 252
-  const dim3 grid((unsigned)ncols), block(c->n_alts + 4);
-  switch (gv::auto_waves(c->n_alts)) {
-    case 1: hipLaunchKernelGGL(sources_kernel<64>, grid, block, lds, h->stream, p, *c, f); break;
-    case 2: hipLaunchKernelGGL(sources_kernel<128>, grid, block, lds, h->stream, p, *c, f); break;
-    case 3: hipLaunchKernelGGL(sources_kernel<192>, grid, block, lds, h->stream, p, *c, f); break;
-    case 4: hipLaunchKernelGGL(sources_kernel<256>, grid, block, lds, h->stream, p, *c, f); break;
+  const size_t lds = ((size_t)W_LEN * row_len(c->n_alts) + PAD + 3) * sizeof(double);  // 91 KB at 252
+  const int waves = gv::auto_waves(c->n_alts);
+  const dim3 grid((unsigned)ncols), block(64 * waves);
+  switch (waves) {
+    case 1: hipLaunchKernelGGL(sources_kernel<64>, grid, block, lds, h->stream, args); break;
+    case 2: hipLaunchKernelGGL(sources_kernel<128>, grid, block, lds, h->stream, args); break;
+    case 3: hipLaunchKernelGGL(sources_kernel<192>, grid, block, lds, h->stream, args); break;
+    case 4: hipLaunchKernelGGL(sources_kernel<256>, grid, block, lds, h->stream, args); break;
     default: return GITM_VERT_EINVAL;
   }
   GV_HIP(hipGetLastError());

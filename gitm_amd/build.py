@@ -23,8 +23,9 @@ HIPFLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-I" + os.path.join(ROOT, "include"), "-I" + CSRC,
 ]
-# The AUSM kernels' stage loop: hoisting its constants out of the loop costs
-# more registers than a lane has, and each is then reloaded from memory.
+# The AUSM kernels' and the adjoint's stage loops: hoisting their constants out
+# of the loop costs more registers than a lane has, and each is then reloaded
+# from memory.
 NO_HOIST = ("-mllvm", "-disable-machine-licm")
 # translation units, compiled in parallel: the single-grid step and C ABI,
 # the ensemble batches (host side, and the step kernel once per workgroup
@@ -34,7 +35,7 @@ SOURCES = (("gitm_vert.hip", (), ""), ("gitm_vert_ausm.hip", NO_HOIST, ""),
            ("gitm_vert_batch.hip", (), ""),
            *(("gitm_vert_ensemble.hip", (f"-DGV_ENS_WAVES={w}",), f"_w{w}")
              for w in (1, 2, 3, 4)),
-           ("gitm_vert_adjoint.hip", (), ""), ("gitm_vert_sources.hip", (), ""),
+           ("gitm_vert_adjoint.hip", NO_HOIST, ""), ("gitm_vert_sources.hip", (), ""),
            ("gitm_horiz.hip", (), ""))
 
 

@@ -1488,7 +1488,10 @@ struct Column {
           BNVm = BNVm + dq((RSL[s] + RSR[s]) * NV, RLR, iRLR);
         }
       }
-      if constexpr (ctx_taps<Ctx>::value) cx.tap_nv(nvp, nvm);
+      if constexpr (ctx_taps<Ctx>::value) {
+        cx.tap_nv(nvp, nvm);
+        cx.tap_sums(RL, RR, PL, PR, VUL, VUR, BNVp, BNVm);
+      }
       // energy and momentum fluxes (:1973-2026)
       if (BNVp >= 0.0) {
         EFp = (EL + PL) * BNVp;

@@ -406,7 +406,7 @@ class VerticalSolver:
         with UAM_Gradient's coefficients "grad_lon" and "grad_lat"
         ([block][M, 0, P][cell]).  ``use_topography`` reads "dalt",
         "dalt_dlon" and "dalt_dlat" (state-shaped) and advances the levels
-        in order, one launch each."""
+        in order, in one launch."""
         import torch
 
         for k, t in grid.items():

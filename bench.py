@@ -522,7 +522,7 @@ def bench_horizontal(torch, solver, reps: int = 10) -> dict:
     xbytes = 2 * 8 * 19 * halo * spec.nalts * spec.nblocks
     nbytes = horizontal_bytes_per_slab(spec.nlons, spec.nlats) * slabs
     del g
-    return {"kernel": "horiz_kernel<17, false> (gitm_horiz_advance: advance_horizontal, RK4 of "
+    return {"kernel": "horiz_flat_kernel (gitm_horiz_advance: advance_horizontal, RK4 of "
                       "the Rusanov/MC lat-lon solver)",
             "workload": "1deg_blocks_800x100: 360x180 cells in 800 blocks of 9x9, "
                         "100 levels, Coriolis on, ions off",
@@ -530,7 +530,7 @@ def bench_horizontal(torch, solver, reps: int = 10) -> dict:
             "achieved": nbytes / (ms * 1e-3) / 1e9, "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": nbytes / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS,
             "cell_updates_per_s": spec.ncells * spec.nalts / (ms * 1e-3),
-            "topography": {"kernel": "horiz_kernel<17, true>, one launch per level",
+            "topography": {"kernel": "horiz_topo_kernel, one launch",
                            "ms_per_step": tms,
                            "cell_updates_per_s": spec.ncells * spec.nalts / (tms * 1e-3)},
             "exchange": {"kernel": "exchange_kernel + exchange_check_kernel "
@@ -745,8 +745,8 @@ def main() -> int:
                      "interface_bytes_per_launch":
                          interface_bytes_per_column(spec.nalts) * ncols,
                      "launch_ms": launch_ms,
-                     "kernel": f"vert_column_kernel<{64 * vertical.auto_waves(spec.nalts)},"
-                               f"{1 if args.solver == 'ausm' else 0}>"},
+                     "kernel": "vert_group_kernel" if args.solver == "ausm" else
+                               f"vert_column_kernel<{64 * vertical.auto_waves(spec.nalts)},0>"},
         "roofline_fp64": roofline_fp64(spec, launch_ms) if args.solver == "ausm" else None,
         "cpu_baseline": cpu,
         "cpu_reference": cpu_ref,

@@ -52,15 +52,6 @@ __device__ __forceinline__ double *hf(const gitm_vert_field &f, int lon, int lat
          (long long)b * f.s_blk;
 }
 
-// Limiter_mc (ModLimiter.f90:16-36) without branches: with both slopes of one
-// sign the smallest of beta |up|, beta |dn|, |up + dn| / 2 with that sign, else
-// zero.
-__device__ __forceinline__ double limiter(double beta, double up, double dn) {
-  const double m = fmin(beta * fmin(fabs(up), fabs(dn)), fabs((up + dn) * 0.5));
-  const long long su = __builtin_bit_cast(long long, up), sd = __builtin_bit_cast(long long, dn);
-  return ((su ^ sd) < 0) ? 0.0 : __builtin_copysign(m, dn);
-}
-
 // The geometry of one cell i (1..n) along one line: InvD*Dist_FB at faces
 // i-1..i+2, d*Dist_FB at faces i and i+1, InvD*Dist_GB(i), half the larger
 // cMax of the cells on either side of faces i and i+1, and whether the cell
@@ -90,7 +81,8 @@ __device__ __forceinline__ void rusanov_cell(const P v, int S, const LineGeo &g,
   double f3 = (g.ifb[3] * 2) * (F1 * dp - F2 * (v3 - v0));
   f0 = g.first ? dm * g.ifb[0] : f0;
   f3 = g.last ? dp * g.ifb[3] : f3;
-  const double s0 = limiter(beta, f1, f0), s1 = limiter(beta, f2, f1), s2 = limiter(beta, f3, f2);
+  const double s0 = gv::limiter_sel(beta, f1, f0), s1 = gv::limiter_sel(beta, f2, f1),
+               s2 = gv::limiter_sel(beta, f3, f2);
   const double l0 = vm1 + 0.5 * s0 * g.dfb0, r0 = v0 - 0.5 * s1 * g.dfb0;
   const double l1 = v0 + 0.5 * s1 * g.dfb1, r1 = v1 - 0.5 * s2 * g.dfb1;
   grad = 0.5 * (l1 + r1 - l0 - r0) * g.igb;

@@ -307,6 +307,35 @@ GV_FN R limiter_mc(double beta, R up, R dn) {
   return 0.0;
 }
 
+// limiter_mc of doubles without branches, for the device: with both slopes of one
+// sign the smallest of beta |up|, beta |dn|, |up + dn| / 2 with that sign, else
+// zero.  p and q are the slopes times the sign of dn, so that the smallest is
+// negative where the signs differ.  A NaN slope counts as in limiter_mc on the
+// device, whose comparisons it fails and whose minima it drops out of: as dn it
+// gives zero (q = 0), as up it leaves beta dn below zero and else zero (u =
+// -inf); a NaN thus changes no slope but its own cell's.
+// The 1-degree horizontal step takes 4.18 ms and the 1-degree AUSM step 11.60 ms;
+// with comparisons of the slopes, which become branches, 4.43 and 11.96 ms; blind
+// to NaN, by the sign bits, 4.17 and 11.51 ms.
+GV_FN double limiter_flat(double beta, double up, double dn) {
+  constexpr unsigned long long SIGN = 1ULL << 63;
+  const double u = __builtin_fmax(up, -__builtin_inf());
+  const unsigned long long p =
+      __builtin_bit_cast(unsigned long long, u) ^ (__builtin_bit_cast(unsigned long long, dn) & SIGN);
+  const double P = __builtin_bit_cast(double, p), q = __builtin_fmax(fabs(dn), 0.0);
+  const double m = __builtin_fmin(beta * __builtin_fmin(P, q), (P + q) * 0.5);
+  return __builtin_copysign(__builtin_fmax(m, 0.0), dn);
+}
+// The limiter of the kernels that take doubles only: limiter_flat on the
+// device, limiter_mc in the host build, which stays bit for bit with the oracle.
+GV_FN double limiter_sel(double beta, double up, double dn) {
+#ifdef GV_HOST_EMULATION
+  return limiter_mc(beta, up, dn);
+#else
+  return limiter_flat(beta, up, dn);
+#endif
+}
+
 // Which value Limiter_mc took: 0 (zero), 1 (beta*up), 2 (beta*dn) or 3
 // ((up+dn)/2), as limiter_mc decides it (the adjoint build records it).
 template <class R>

@@ -137,21 +137,6 @@ GV_FN double quot(double a, double d) {
 #endif
 }
 
-// Limiter_mc (ModLimiter.f90:16-36) without branches: with both slopes of one
-// sign the smallest of beta |up|, beta |dn|, |up + dn| / 2 with that sign,
-// else zero (the bits of limiter_mc, and like it no NaN from a NaN slope).
-// Five FP64 and five 32-bit instructions; the two nested branches of
-// limiter_mc cost about twice that when a wavefront holds both signs.
-GV_FN double limiter_sel(double beta, double up, double dn) {
-#ifdef GV_HOST_EMULATION
-  return limiter_mc(beta, up, dn);
-#else
-  const double m = dmin(beta * dmin(fabs(up), fabs(dn)), fabs((up + dn) * 0.5));
-  const long long su = __builtin_bit_cast(long long, up), sd = __builtin_bit_cast(long long, dn);
-  return ((su ^ sd) < 0) ? 0.0 : __builtin_copysign(m, dn);
-#endif
-}
-
 // The friction solve of one level (calc_neutral_friction.f90:47-106):
 // (1 + dt sum_q C_iq) x_i - dt sum_q C_iq x_q = w_i with C_iq = k T n_q /
 // (m_i N D_iq).  Row i times m_i n_i makes the system symmetric,

@@ -1019,7 +1019,9 @@ struct GroupColumn {
         Ai[q] = 0.0;
       }
     }
-    const double idt = 1.0 / dt;
+    // dt may be 0 (a member's step from the prep, at EndTime): what it divides
+    // is then so large that MPn is 0, and recip takes no infinite operand
+    const double idt = dmax(-0x1p300, dmin(1.0 / dt, 0x1p300));
 #pragma unroll 1
     for (int stg = 0; stg < 4; stg++) {
       stage(stg == 2 ? dt : 0.5 * dt, stg == 2 ? idt : 2.0 * idt, stg);  // :160-377

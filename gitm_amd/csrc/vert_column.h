@@ -116,12 +116,17 @@ constexpr int DEXI[NSP][NSP] = {{0, 0, 0, 0, 1, 2},
 // :1052-1053); Factor2 is the literal 0.0416667, not 1/24.
 constexpr double FACT1 = 0.6250000, FACT2 = 0.0416667;
 
+// A power of two that the masses and kT of the friction system are multiplied by
+// (see friction_solve, vert_group.h).
+constexpr double FRIC_SCALE = 70368744177664.0;  // 2^46
+
 // Kernel-side run constants (built on the host from gitm_vert_params).
 struct KParams {
   double dt, beta, maxvv, min_tec, vert_tau, omega;
   double mass[NSP], tdc[NSP];
   double lmass[NSP];  // log(mass), for the log-space forms of the device math
   double imass[NSP];  // 1/mass, ditto
+  double fmass[NSP];  // FRIC_SCALE mass, for the friction system of vert_group.h
   double log_min_kp, log_max_kp, log_min_ku, log_max_ku;  // log(1e-19), ...
   int n_alts, n_steps, solver;
   int friction, coriolis, ions, improved_ions, nighttime_ion_bcs;

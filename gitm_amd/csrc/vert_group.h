@@ -137,21 +137,35 @@ GV_FN double quot(double a, double d) {
 #endif
 }
 
+// What MPn's numerator (in Kp) and denominator (in the mean density) are
+// multiplied by: the denominator of a species of 1e-283 per m^3 is then far from
+// the end of the range, where recip overflows.  A power of two: the same bits.
+constexpr double MP_SCALE = 0x1p100;
+
 // The friction solve of one level (calc_neutral_friction.f90:47-106):
 // (1 + dt sum_q C_iq) x_i - dt sum_q C_iq x_q = w_i with C_iq = k T n_q /
 // (m_i N D_iq).  Row i times m_i n_i makes the system symmetric,
 // A_iq = -dt k T n_i n_q / (N D_iq), and A_ii = m_i n_i - sum_q A_iq: positive
 // definite and diagonally dominant, so the LDL^T factors need no pivoting and
-// half the operations.  pw[u] = T**-DEXU[u].  Returns the sum of the x_i: finite
-// unless something in the system is not.
-GV_FN double friction_solve(const KParams &P, double dt, const double (&ns)[NSP], double T,
-                            const double (&pw)[6], double (&w)[NSP]) {
-  const double dkT = dt * (KB * T);
-  double a[NSP][NSP], e[6];  // the upper triangle
+// half the operations.  pw[u] = T**-DEXU[u], nt the sum of the n_i.  Returns the
+// sum of the x_i: finite unless something in the system is not.
+// The whole system is multiplied by a power of two, 2^110 over about nt: the
+// m_i n_i of a minor species and the n_i n_q would leave the range (densities
+// below 1e-282 or above 1e150 per m^3), and the solution does not change a bit.
+GV_FN double friction_solve(const KParams &P, double dt, const double (&ns)[NSP], double nt,
+                            double T, const double (&pw)[6], double (&w)[NSP]) {
+  const double dkT = dt * ((FRIC_SCALE * KB) * T);
+  int ex;
+  frexp_mant(nt, ex);
+  const double unit = ldexp(1.0, 64 - (ex < -900 ? -900 : ex));
+  double a[NSP][NSP], e[6], nu[NSP];  // the upper triangle
 #pragma unroll
   for (int u = 0; u < 6; u++) e[u] = dkT * pw[u];
 #pragma unroll
-  for (int i = 0; i < NSP; i++) a[i][i] = P.mass[i] * ns[i];
+  for (int i = 0; i < NSP; i++) {
+    nu[i] = ns[i] * unit;
+    a[i][i] = P.fmass[i] * nu[i];
+  }
 #pragma unroll
   for (int i = 0; i < NSP; i++) w[i] = a[i][i] * w[i];
 #pragma unroll
@@ -159,7 +173,7 @@ GV_FN double friction_solve(const KParams &P, double dt, const double (&ns)[NSP]
 #pragma unroll
     for (int q = i + 1; q < NSP; q++) {
       const double g = 1.0e-19 / D0R[i][q];  // 1e-2 / Diff0, a constant
-      const double c = (ns[i] * ns[q]) * (g * e[DEXI[i][q]]);
+      const double c = (nu[i] * ns[q]) * (g * e[DEXI[i][q]]);
       a[i][q] = -c;
       a[i][i] = a[i][i] + c;
       a[q][q] = a[q][q] + c;
@@ -312,7 +326,7 @@ struct GroupColumn {
       double vp = 0.0, vu = 0.0;
       if (cell()) {
         const double th = (1.0 + tanh((alt - 160.0e+03) / 15.0e+03));
-        vp = exp(kp.log_min_kp + 0.5 * (kp.log_max_kp - kp.log_min_kp) * th);
+        vp = MP_SCALE * exp(kp.log_min_kp + 0.5 * (kp.log_max_kp - kp.log_min_kp) * th);
         vu = exp(kp.log_min_ku + 0.5 * (kp.log_max_ku - kp.log_min_ku) * th);
       }
       x(GR_KP, j) = vp;
@@ -807,7 +821,7 @@ struct GroupColumn {
 #pragma unroll
       for (int q = 0; q < SPW; q++) {
         const double MPS = 0.5 * (PSL[q] + PSR[q]), MHPS = 0.5 * (HL[q] + HR[q]);
-        const double RS2 = RSL[q] + RSR[q], MRS = 0.5 * RS2;
+        const double RS2 = RSL[q] + RSR[q], MRS = (0.5 * MP_SCALE) * RS2;
         const double ML = VL[q] * icS, MR = VR[q] * icS;  // :1689-1706
         const double M2 = 0.5 * (ML * ML + MR * MR);
         const double MZ = sqrt(dmin(1.0, dmax(M2, 1.0e-19)));
@@ -904,7 +918,7 @@ struct GroupColumn {
         nrs[q] = rhos[q] - dtin * rsf;
         const double src = ((sub >> q) & 1) ? dev[q] : rhos[q];
         const double nm = rhos[q] * W0[q] - dtin * msf + dtin * src * eg;
-        double ww = quot(nm, nrs[q]);
+        double ww = nm / nrs[q];  // (nrs may lie below quot's range)
         ww = ww + dtin * (vn * vn + ve * ve) * at(GR_INVR);
         if (kp.coriolis) ww = ww + dtin * (sc(GS_COR) * ve);
         ww = ww - dtin * (kp.tdc[s0 + q] * KB * gradT) * im;
@@ -939,7 +953,7 @@ struct GroupColumn {
         }
         nnt = ((ns[0] + ns[1]) + (ns[2] + ns[3])) + (ns[4] + ns[5]);
         if (kp.friction) {
-          const double sum = friction_solve(kp, dtin, ns, at(GU_T), pw, w);
+          const double sum = friction_solve(kp, dtin, ns, nnt, at(GU_T), pw, w);
           if (!(fabs(sum) < __builtin_inf()) && friction_singular(&at(GU_LN), at(GU_T)))
             fail(GITM_VERT_ESINGULAR, k);
 #pragma unroll

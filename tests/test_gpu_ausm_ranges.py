@@ -1,6 +1,8 @@
 """The AUSM step at the ends of what it accepts, against the oracle within the
 step's parity bar, 1e-11: time steps of zero (a batch member's, from the prep at
-the end of the run) and far below a second."""
+the end of the run) and far below a second; a species, or all of them, in
+densities whose masses, products or reciprocals come near the ends of the double
+range."""
 from __future__ import annotations
 
 import dataclasses
@@ -50,3 +52,26 @@ def test_short_steps(solver, dt):
     solver.advance(d, p, "ausm", 1)
     assert_parity(vertical.to_host(d), cpu.advance(cols, p, solver=1, threads=THREADS), 1e-11,
                   what=f"dt {dt}")
+
+
+@pytest.mark.parametrize("species,factor", [(0, 1e-250), (0, 1e-290), (0, 1e-300), (5, 1e-300),
+                                            (None, 1e-290), (None, 1e-200), (None, 1e100),
+                                            (None, 1e140), (None, 1e200), (None, 1e250)])
+def test_densities_far_from_one(solver, species, factor):
+    """1e-300 of a species leaves mass densities of 1e-309; 1e140 of all gives
+    products of two densities beyond 1e308."""
+    from gitm_amd import vertical
+    cols = columns(50, 42)
+    odd = np.arange(cols["temp"].shape[0]) % 2 == 1
+    if species is None:
+        cols["nds"][odd] *= factor
+        cols["rho"][odd] *= factor
+    else:
+        cols["nds"][odd, species] *= factor
+    p = synth.StepParams()
+    with np.errstate(all="ignore"):
+        ref = cpu.advance(cols, p, solver=1, threads=THREADS)
+    d = vertical.to_device(cols)
+    print(f"species {species} x {factor}", flush=True)
+    solver.advance(d, p, "ausm", 1)
+    assert_parity(vertical.to_host(d), ref, 1e-11, what=f"species {species} x {factor}")

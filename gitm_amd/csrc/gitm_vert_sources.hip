@@ -11,10 +11,11 @@
 // multiplication by a rounded reciprocal will do; what is left is to make
 // the serial part short and to keep enough columns on a CU to hide it:
 //  * the quotients are the hardware's own division sequence without its
-//    scaling and special cases (div_neg), whose reciprocal a pivot's two
-//    quotients share; range tests beside the chains tell whether that was
-//    exact, and a column where it may not have been is done again with plain
-//    divisions;
+//    scaling and special cases (vert_sources_chain.h), whose reciprocal a
+//    pivot's two quotients share; range tests beside the chains tell whether
+//    that was exact, and a column where it may not have been is done again with
+//    plain divisions.  Zeros pass: after a vertical step the east and north
+//    winds of level 0 are zero in every column;
 //  * a chain reads ahead, two levels per LDS access (rows of the LDS image
 //    run along altitude), and holds little but its arithmetic: per level the
 //    first sweeps take 150 clocks, of which 88 are the serial operations, the
@@ -28,11 +29,15 @@
 // 34 of a column's 65 thousand clocks (LDS writes of 26 clocks each on top of
 // the arithmetic), with 1.6 TB/s of HBM in use.  64,800 columns of 100 levels
 // took 3.25 ms with a division in each link of the chains, 63 doubles per
-// level and no read ahead; they take 1.72 ms.  A column done again costs what
-// it cost then: the plain pass has no read ahead, but four columns per CU.
+// level and no read ahead; they take 1.74 ms, before and after a vertical step.
+// Were all of them done again it would be 3.7 ms: the quick pass up to the test
+// that fails, then a plain one without read ahead.
 #include "vert_gpu.h"
+#include "vert_sources_chain.h"
 
 namespace {
+
+using namespace gv::chain;
 
 struct SrcParams {
   double dt;
@@ -84,75 +89,6 @@ static_assert(2 * NQ <= 64, "both solves' lanes in one wavefront");
 // 16-byte aligned, and odd in pairs, so that the chain lanes' rows fall on
 // different LDS banks.
 constexpr int row_len(int n_alts) { return (n_alts + 4) + ((2 - (n_alts + 4)) & 3); }
-
-// IEEE division without its range handling.  The hardware's sequence is:
-// scale both operands, refine v_rcp_f64 twice, multiply, correct by the
-// remainder, undo the scaling and fix special operands up.  The scalings are
-// by powers of two, so where neither the operands nor the remainder leave the
-// normal range the middle part alone gives the same bits: div_recip's refined
-// reciprocal, which quotients by one divisor share, and a multiplication and
-// correction.  div_pos is for divisors > 0 and div_neg for divisors < 0: they
-// differ in the sign of a zero remainder, which makes the quotients of +0 and
-// -0 right too.
-__device__ __forceinline__ double div_recip(double d) {
-  double r = __builtin_amdgcn_rcp(d);
-  r = __builtin_fma(__builtin_fma(-d, r, 1.0), r, r);
-  return __builtin_fma(__builtin_fma(-d, r, 1.0), r, r);
-}
-__device__ __forceinline__ double div_pos(double n, double d, double r) {
-  const double q = n * r;
-  return __builtin_fma(-__builtin_fma(d, q, -n), r, q);
-}
-__device__ __forceinline__ double div_neg(double n, double d, double r) {
-  const double q = n * r;
-  return __builtin_fma(__builtin_fma(-d, q, n), r, q);
-}
-
-// Whether the quick divisions may be used is decided by range.  Divisors
-// known before the chains are positive and within 2^-200..2^200, numerators
-// zero or within 2^-200..2^200, matrix elements within 2^200; the pivots are
-// negative and within 2^-256..2^256 (Pivots), the forward sweeps' values
-// zero throughout or above 2^-600 throughout, and what comes out finite.
-// Otherwise the column is done again with plain divisions.
-struct Range {
-  double lo = 0x1p200, hi = 0.0;  // of the divisors, and of every magnitude
-  bool tiny = false;
-  __device__ __forceinline__ void divisor(double x) {
-    lo = fmin(lo, x);
-    hi = fmax(hi, x);
-  }
-  __device__ __forceinline__ void element(double x) { hi = fmax(hi, fabs(x)); }
-  __device__ __forceinline__ void numerator(double x) {
-    element(x);
-    tiny |= (x != 0.0) & (fabs(x) < 0x1p-200);
-  }
-  __device__ bool good() const { return (lo > 0x1p-200) & (hi < 0x1p200) & !tiny; }
-};
-
-// The ranges of a chain's pivots and values, from the high words of two
-// levels at once (as integers negative doubles ascend with their magnitude;
-// as floats the words' magnitudes compare as the doubles').
-struct Pivots {
-  int lo = 0x7fffffff, hi = (int)0x80000000;
-  __device__ __forceinline__ void see(double x, double y) {
-    lo = min(min(__double2hiint(x), __double2hiint(y)), lo);
-    hi = max(max(__double2hiint(x), __double2hiint(y)), hi);
-  }
-  __device__ bool good() const {
-    return lo >= __double2hiint(-0x1p-256) && hi < __double2hiint(-0x1p256);
-  }
-};
-struct Values {
-  float lo = __builtin_huge_valf(), hi = 0.0f;
-  __device__ __forceinline__ void see(double x, double y) {
-    const float u = __int_as_float(__double2hiint(x)), v = __int_as_float(__double2hiint(y));
-    asm("v_min3_f32 %0, %0, |%1|, |%2|" : "+v"(lo) : "v"(u), "v"(v));
-    asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(hi) : "v"(u), "v"(v));
-  }
-  __device__ bool good() const {
-    return hi == 0.0f || lo >= __int_as_float(__double2hiint(0x1p-600));
-  }
-};
 
 struct SrcCol {
   const SrcArgs *args;
@@ -221,7 +157,7 @@ __device__ __forceinline__ Coef coefficients(Range &range, int k, int nA, double
     range.numerator(dl);
     range.numerator(told);
     range.numerator(o.c);
-    range.element(o.a);
+    range.numerator(o.a);
     range.element(o.ba);
     range.element(o.bc);
   }
@@ -237,217 +173,6 @@ __device__ __forceinline__ Coef coefficients(Range &range, int k, int nA, double
   }
   if (k < 1 || top) o.d = -told;
   return o;
-}
-
-// Two levels of a row from level i on, i odd: 16-byte aligned.
-__device__ __forceinline__ double2 load2(const double *row, int i) {
-  return *reinterpret_cast<const double2 *>(row + i);
-}
-__device__ __forceinline__ void store2(double *row, int i, double2 v) {
-  *reinterpret_cast<double2 *>(row + i) = v;
-}
-
-// The chains take two levels at a time.  A lone wavefront issues one
-// instruction of whatever kind every 4 to 5 clocks and an LDS read takes some
-// 60, so the loops hold nothing but arithmetic, 16-byte LDS accesses and an
-// address per row: a ring of P pairs holds operands on their way, a pair's
-// slot is read anew as soon as its levels are done, U rounds of the ring are
-// unrolled, and what is read past the last pair (within the LDS image, PAD
-// doubles beyond its last row) is not used.  step(slot, i) works on levels i
-// and i + 1 and read(slot, i) starts its reads; n pairs from level i0 on in
-// steps of d levels.
-template <int P, int U, class Slot, class Read, class Step>
-__device__ __forceinline__ void ring(int n, int i0, int d, const Read &read, const Step &step) {
-  Slot x[P];
-#pragma unroll
-  for (int p = 0; p < P; p++) read(x[p], i0 + p * d);
-  int i = i0;
-  for (; n >= P * U; n -= P * U, i += P * U * d) {
-#pragma unroll
-    for (int p = 0; p < P * U; p++) {
-      step(x[p % P], i + p * d);
-      GV_ORDER();
-      read(x[p % P], i + (p + P) * d);
-      GV_ORDER();
-    }
-  }
-#pragma unroll
-  for (int p = 0; p < P * U - 1; p++)
-    if (p < n) {
-      step(x[p % P], i + p * d);
-      if (p + P < P * U - 1) read(x[p % P], i + (p + P) * d);
-    }
-}
-constexpr int PAD = 16;  // ring reads at most P pairs past the last level
-
-// The forward sweep of one solve (:232-241): cp to rb, dp to wd.  sc d is the
-// solve's right side (sc is 1 or 2: the fma rounds once).
-struct Fwd {
-  double2 a, c, b, d;
-};
-// cp at one level, and dp at the level below, whose pivot is known by then:
-// dp's five operations go between those of the pivot's reciprocal, each of
-// which waits 6 to 22 clocks for the one before (88 a level).
-struct Forward {
-  double sc, cp, dp;
-  double a, d, den, r;  // the level below's
-  __device__ __forceinline__ void level(double a1, double c1, double b1, double d1) {
-    const double t = cp * a1;
-    GV_ORDER();
-    const double den1 = b1 - t;
-    const double u = dp * a;
-    GV_ORDER();
-    const double r0 = __builtin_amdgcn_rcp(den1);
-    const double n = __builtin_fma(d, sc, -u);
-    GV_ORDER();
-    const double q = n * r;
-    const double e0 = __builtin_fma(-den1, r0, 1.0);
-    GV_ORDER();
-    const double m = __builtin_fma(-den, q, n);
-    const double r1 = __builtin_fma(e0, r0, r0);
-    GV_ORDER();
-    dp = __builtin_fma(m, r, q);
-    const double e1 = __builtin_fma(-den1, r1, 1.0);
-    GV_ORDER();
-    const double r2 = __builtin_fma(e1, r1, r1);
-    const double qc = c1 * r2;
-    const double mc = __builtin_fma(-den1, qc, c1);
-    cp = __builtin_fma(mc, r2, qc);
-    a = a1;
-    d = d1;
-    den = den1;
-    r = r2;
-  }
-  __device__ __forceinline__ double last() {
-    const double n = __builtin_fma(d, sc, -(dp * a));
-    return dp = div_neg(n, den, r);
-  }
-};
-template <bool FAST>
-__device__ __forceinline__ bool sweep(const double *ra, const double *rc, double *rb,
-                                      const double *rd, double *wd, double sc, int nA, double &cp,
-                                      double &dp) {
-  const auto plain = [&](double a, double c, double b, double d) {
-    const double den = b - cp * a;
-    const double n = __builtin_fma(d, sc, -(dp * a));
-    cp = c / den;
-    dp = n / den;
-    return den;
-  };
-  if (!FAST) {
-    for (int i = 1; i <= nA; i++) {
-      plain(ra[i], rc[i], rb[i], rd[i]);
-      rb[i] = cp;
-      wd[i] = dp;
-    }
-    return true;
-  }
-  Pivots pivots;
-  Values values;
-  // the odd level out, if there is one, is read before the ring runs
-  const double a1 = ra[nA], c1 = rc[nA], b1 = rb[nA], d1 = rd[nA];
-  // the level below level 1 gives dp = dp(0)
-  Forward f{sc, cp, 0.0, 0.0, -dp / sc, -1.0, -1.0};
-  double v0 = dp;
-  ring<2, 4, Fwd>(
-      nA / 2, 1, 2,
-      [&](Fwd &x, int i) {
-        x.b = load2(rb, i);
-        x.a = load2(ra, i);
-        x.c = load2(rc, i);
-        x.d = load2(rd, i);
-      },
-      [&](Fwd &x, int i) {
-        double2 c;
-        f.level(x.a.x, x.c.x, x.b.x, x.d.x);
-        const double p0 = f.den;
-        c.x = f.cp;
-        const double v1 = f.dp;
-        f.level(x.a.y, x.c.y, x.b.y, x.d.y);
-        c.y = f.cp;
-        store2(rb, i, c);
-        store2(wd, i - 2, make_double2(v0, v1));
-        pivots.see(p0, f.den);
-        values.see(v0, v1);
-        v0 = f.dp;
-      });
-  const int top = nA & ~1;
-  cp = f.cp;
-  dp = f.last();
-  values.see(v0, dp);
-  store2(wd, top - 1, make_double2(v0, dp));
-  if (nA & 1) {
-    const double p = plain(a1, c1, b1, d1);
-    pivots.see(p, p);
-    values.see(dp, dp);
-    rb[nA] = cp;
-    wd[nA] = dp;
-  }
-  return pivots.good() && values.good();
-}
-
-// The forward sweep on known pivots: dp over the right side in rn.
-struct Fwd2 {
-  double2 a, n, den, r;
-};
-template <bool FAST>
-__device__ __forceinline__ bool sweep2(const double *ra, double *rn, const double *rden,
-                                       const double *rr, int nA, double &dp) {
-  if (!FAST) {
-    for (int i = 1; i <= nA; i++) rn[i] = dp = (rn[i] - dp * ra[i]) / rden[i];
-    return true;
-  }
-  Values values;
-  const double a1 = ra[nA], n1 = rn[nA], den1 = rden[nA];
-  ring<3, 2, Fwd2>(
-      nA / 2, 1, 2,
-      [&](Fwd2 &x, int i) {
-        x.a = load2(ra, i);
-        x.n = load2(rn, i);
-        x.r = load2(rr, i);
-        x.den = load2(rden, i);
-      },
-      [&](Fwd2 &x, int i) {
-        double2 v;
-        v.x = dp = div_neg(x.n.x - dp * x.a.x, x.den.x, x.r.x);
-        v.y = dp = div_neg(x.n.y - dp * x.a.y, x.den.y, x.r.y);
-        values.see(v.x, v.y);
-        store2(rn, i, v);
-      });
-  if (nA & 1) {
-    rn[nA] = dp = (n1 - dp * a1) / den1;
-    values.see(dp, dp);
-  }
-  return values.good();
-}
-
-// The back substitution (:243-247), levels nA..0: the solution over dp in
-// rd; t the value at nA + 1.
-struct Back {
-  double2 cp, dp;
-};
-template <bool FAST>
-__device__ __forceinline__ void back(const double *rc, double *rd, int nA, double t) {
-  if (!FAST) {
-    for (int i = nA; i >= 0; i--) rd[i] = t = rd[i] - rc[i] * t;
-    return;
-  }
-  const double c0 = rc[0], d0 = rd[0], c1 = rc[nA], d1 = rd[nA];
-  if (nA & 1) rd[nA] = t = d1 - c1 * t;
-  const int n = nA / 2;
-  ring<4, 2, Back>(
-      n, 2 * n - 1, -2,
-      [&](Back &x, int i) {
-        x.cp = load2(rc, i);
-        x.dp = load2(rd, i);
-      },
-      [&](Back &x, int i) {
-        double2 v;
-        v.y = t = x.dp.y - x.cp.y * t;
-        v.x = t = x.dp.x - x.cp.x * t;
-        store2(rd, i, v);
-      });
-  rd[0] = d0 - c0 * t;
 }
 
 // A level's values that outlive the solves.

@@ -12,9 +12,9 @@
 // gitm_vert_ausm.hip
 void launch_ausm_batch(unsigned ncols, int n_alts, hipStream_t stream, const gv::KParams &kp,
                        const BatchMember *mem, int n, const double *dt_dev);
-void launch_ausm_tall_ions(unsigned ncols, hipStream_t stream, const gv::KParams &kp,
-                           const gitm_vert_columns &c, double *scratch, const double *dt_dev,
-                           int err_first);
+void launch_ausm_tall_ions(unsigned ncols, int n_alts, hipStream_t stream,
+                           const gv::KParams &kp, const BatchMember *mem, int n,
+                           const double *dt_dev);
 
 #define GV_ENS_DECL(W)                                                                     \
   int ensemble_occupancy_w##W(bool ions, size_t lds_bytes);                                \
@@ -99,6 +99,11 @@ struct gitm_vert_batch {
   };
   std::vector<Class> classes[2];  // [ions]
   BatchMember *d_sorted[2] = {};  // first_block counts within the class
+  // with ions: the members (of `table`) that group_fits refuses, in one launch
+  std::vector<int> tall_ions;
+  int tall_ion_alts = 0;
+  long long tall_ion_cols = 0;
+  BatchMember *d_tall_ions = nullptr;  // filled with the layout
   BatchMember *d_table = nullptr;
   double *scratch = nullptr;
   size_t scratch_bytes = 0;
@@ -125,8 +130,19 @@ int ausm_columns_per_cu(int n_alts, bool ions, size_t lds_max) {
 // greater number, and together where they are too few to fill it twice.
 int ausm_classes(gitm_vert_batch *b, bool ions) {
   std::vector<BatchMember> m;
-  for (const BatchMember &e : b->table)
-    if (gv::group_fits(e.io.n_alts, ions)) m.push_back(e);
+  for (int i = 0; i < (int)b->table.size(); i++) {
+    const BatchMember &e = b->table[i];
+    if (gv::group_fits(e.io.n_alts, ions)) {
+      m.push_back(e);
+      continue;
+    }
+    b->tall_ions.push_back(i);
+    b->tall_ion_alts = std::max(b->tall_ion_alts, e.io.n_alts);
+    b->tall_ion_cols += member_columns(e.io);
+  }
+  if (!b->tall_ions.empty() &&
+      hipMalloc(&b->d_tall_ions, b->tall_ions.size() * sizeof(BatchMember)) != hipSuccess)
+    return GITM_VERT_ENOMEM;
   std::stable_sort(m.begin(), m.end(), [](const BatchMember &p, const BatchMember &q) {
     return p.io.n_alts > q.io.n_alts;
   });
@@ -256,6 +272,18 @@ int batch_layout(gitm_vert_batch *b) {
     m.scratch = b->scratch + reinterpret_cast<size_t>(m.scratch);
   GV_HIP(hipMemcpy(b->d_table, dev.data(), dev.size() * sizeof(BatchMember),
                    hipMemcpyHostToDevice));
+  if (!b->tall_ions.empty()) {
+    // (their carries are in the scratch under every tile that fits)
+    std::vector<BatchMember> t;
+    int first = 0;
+    for (int i : b->tall_ions) {
+      t.push_back(dev[i]);
+      t.back().first_block = first;
+      first += (int)member_columns(dev[i].io);
+    }
+    GV_HIP(hipMemcpy(b->d_tall_ions, t.data(), t.size() * sizeof(BatchMember),
+                     hipMemcpyHostToDevice));
+  }
   for (int i = 0; i < 2; i++) {
     b->slot[i] = slot_doubles(b, i != 0, flag);
     b->lds[i] = tile_lds(b, b->tile, i != 0);
@@ -355,6 +383,7 @@ int gitm_vert_batch_destroy(gitm_vert_batch *b) {
   if (b->d_table) (void)hipFree(b->d_table);
   for (BatchMember *s : b->d_sorted)
     if (s) (void)hipFree(s);
+  if (b->d_tall_ions) (void)hipFree(b->d_tall_ions);
   if (b->scratch) (void)hipFree(b->scratch);
   delete b;
   return GITM_VERT_OK;
@@ -396,12 +425,9 @@ int gitm_vert_batch_advance(gitm_vert_batch *b, const gitm_vert_params *p, int s
                         c.n, dt_device);
       GV_HIP(hipGetLastError());
     }
-    for (const BatchMember &e : b->table) {
-      if (gv::group_fits(e.io.n_alts, ions)) continue;
-      // (their carries are in the batch's scratch under every tile that fits)
-      launch_ausm_tall_ions((unsigned)member_columns(e.io), h->stream, kp, e.io,
-                            b->scratch + reinterpret_cast<size_t>(e.scratch),
-                            dt_device ? dt_device + e.member : nullptr, e.col_offset);
+    if (ions && !b->tall_ions.empty()) {
+      launch_ausm_tall_ions((unsigned)b->tall_ion_cols, b->tall_ion_alts, h->stream, kp,
+                            b->d_tall_ions, (int)b->tall_ions.size(), dt_device);
       GV_HIP(hipGetLastError());
     }
     return GITM_VERT_OK;

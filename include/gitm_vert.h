@@ -259,8 +259,8 @@ int gitm_vert_prepare(gitm_vert_handle *h, const gitm_vert_prep_params *p,
  * is stepped exactly as gitm_vert_advance would step it alone.
  *
  * A batch step is one launch over the columns of every member of like height
- * (AUSM: one to four launches), or of every member (Rusanov, see
- * gitm_vert_batch_tile).  gitm_vert_batch_create builds the
+ * (AUSM: one to four launches, and one of the members with ions above 226
+ * levels), or of every member (Rusanov, see gitm_vert_batch_tile).  gitm_vert_batch_create builds the
  * device member table and reserves the scratch memory; afterwards
  * gitm_vert_batch_advance and gitm_vert_batch_prepare only queue kernels on
  * the handle's stream (no allocation, no copy, no synchronisation), so a

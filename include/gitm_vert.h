@@ -207,7 +207,9 @@ int gitm_vert_advance_noalloc(const gitm_vert_params *p, const gitm_vert_columns
 int gitm_vert_get_error(gitm_vert_handle *h, gitm_vert_error *err);
 
 /* Tile choice: waves per column (1..4) for the next launches; 0 restores
- * the automatic choice (smallest that holds nAlts+4 levels). */
+ * the automatic choice (smallest that holds nAlts+4 levels).  The AUSM step
+ * sizes its workgroups by the columns alone; a choice that does not hold
+ * nAlts+4 levels is refused there too. */
 int gitm_vert_set_tile(gitm_vert_handle *h, int waves_per_column);
 
 const char *gitm_vert_strerror(int code);

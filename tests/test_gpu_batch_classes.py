@@ -1,4 +1,5 @@
-"""The launches of a batch's AUSM step: members whose columns have ions and are
+"""The launches of a batch's AUSM step: one per class of column heights, with the
+bits that each member has alone; members whose columns have ions and are
 too tall for the kernel that splits a level over the species take one launch
 together, not one each."""
 from __future__ import annotations
@@ -79,3 +80,25 @@ def test_tall_ion_members_run_side_by_side(solver):
     one, all_ = ms(cols[:1]), ms(cols)
     print(f"one member {one:.3f} ms, sixteen {all_:.3f} ms", flush=True)
     assert all_ < 4.0 * one
+
+
+@pytest.mark.parametrize("ions", [False, True])
+def test_height_classes(solver, ions):
+    """Enough columns of 150 and of 100 levels to fill the chip twice: they and
+    the 50-level members are launches of their own, the second with a member of
+    fewer wavefronts than its workgroups hold; each member with its own step."""
+    import torch
+    from gitm_amd import vertical
+    n_cu = torch.cuda.get_device_properties(0).multi_processor_count
+    tall = -(-2 * n_cu // 81) + 1  # members' blocks of 81 columns
+    layout = [(50, 1), (150, tall), (61, 1), (100, 2 * tall), (20, 1), (12, 1)]
+    cols = [synth.make_columns(synth.GridSpec(nb, 1, na), seed=90 + i, ions=ions)
+            for i, (na, nb) in enumerate(layout)]
+    dts = [2.0, 1.5, 0.5, 1.0, 2.0, 0.25]
+    dev = [vertical.to_device(c) for c in cols]
+    b = vertical.VerticalBatch(solver, dev, ions=ions)
+    p = synth.StepParams(use_ion_advection=ions)
+    print(f"classes, ions {ions}", flush=True)
+    b.advance(p, "ausm", 1, dt=torch.tensor(dts, dtype=torch.float64, device="cuda"))
+    same_as_alone(solver, cols, dev, p, dts)
+    b.close()

@@ -319,9 +319,9 @@ GV_FN R limiter_mc(double beta, R up, R dn) {
 // device, whose comparisons it fails and whose minima it drops out of: as dn it
 // gives zero (q = 0), as up it leaves beta dn below zero and else zero (u =
 // -inf); a NaN thus changes no slope but its own cell's.
-// The 1-degree horizontal step takes 4.18 ms and the 1-degree AUSM step 11.60 ms;
-// with comparisons of the slopes, which become branches, 4.43 and 11.96 ms; blind
-// to NaN, by the sign bits, 4.17 and 11.51 ms.
+// Against a selection by the slopes' sign bits, which is blind to NaN, it costs 0.8 %
+// of the 1-degree AUSM step and 0.3 to 1.4 % of the horizontal steps; comparisons
+// of the slopes, which become branches, cost 4 and 6 %.
 GV_FN double limiter_flat(double beta, double up, double dn) {
   constexpr unsigned long long SIGN = 1ULL << 63;
   const double u = __builtin_fmax(up, -__builtin_inf());

@@ -603,15 +603,15 @@ struct GroupColumn {
   // States of face k|k+1 of a field with the values fm1, f0, f1, f2 on levels
   // k-1..k+2 (calc_kt_facevalues, :2073-2117).
   struct FaceGeo {
-    double iF0, iF1, iF2, dF0, dF1;
+    double iF0, iF1, iF2, hF0, hF1;  // hF: half the distances below and above
   };
   GV_MEM void kt(const FaceGeo &q, double fm1, double f0, double f1, double f2, double &l,
                  double &r) const {
     const double mid = (f1 - f0) * q.iF1;
     const double d0 = limiter_sel(kp.beta, mid, (f0 - fm1) * q.iF0);
     const double d1 = limiter_sel(kp.beta, (f2 - f1) * q.iF2, mid);
-    l = f0 + 0.5 * d0 * q.dF0;
-    r = f1 - 0.5 * d1 * q.dF1;
+    l = f0 + d0 * q.hF0;
+    r = f1 - d1 * q.hF1;
   }
 
   // advance_vertical_1stage_ausm (vertical_solver_ausm.f90:436-999) with
@@ -737,7 +737,8 @@ struct GroupColumn {
     double RSL[SPW], RSR[SPW], PSL[SPW], PSR[SPW], HL[SPW], HR[SPW], VL[SPW], VR[SPW];
     const int subUp = reinterpret_cast<int &>(own(GP_SUB, 1));  // flags of cell k+1
     {
-      const FaceGeo fg = {at(GR_IF), at(GR_IF, 1), at(GR_IF, 2), at(GR_DF), at(GR_DF, 1)};
+      const FaceGeo fg = {at(GR_IF), at(GR_IF, 1), at(GR_IF, 2), 0.5 * at(GR_DF),
+                          0.5 * at(GR_DF, 1)};
       double mL = 0.0, mR = 0.0;
 #pragma unroll
       for (int q = 0; q < SPW; q++) {

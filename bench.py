@@ -46,15 +46,18 @@ if ROOT not in sys.path:
 WORKLOAD = "1deg_64800x100"
 HBM_PEAK_GBS = 8000.0
 FP64_PEAK_TFLOPS = 78.6
-TRAFFIC_FILE = os.path.join(ROOT, "profiles", "vert_column_ausm_1deg_64800x100_traffic.txt")
+TRAFFIC_FILE = os.path.join(ROOT, "profiles", "vert_group_ausm_1deg_64800x100_traffic.txt")
 
 
-# FP64 operations of one AUSM column-update as the product column code does
-# them (device forms; faces once; every lane of the column, idle tile lanes
-# excluded), counted by class by running that code over a counting number
-# type on the host (tests/emu/count.h; tests/test_flop_count.py recomputes
-# them): column 0 of the seeded 1-degree workload (nAlts 100) and of the
-# 5-degree one (nAlts 50).  Columns differ by about 0.1% (branches).
+# FP64 operations of one AUSM column-update as the column code with one lane per
+# level does them (vert_column.h: device forms; faces once; every lane of the
+# column, idle tile lanes excluded), counted by class by running that code over a
+# counting number type on the host (tests/emu/count.h; tests/test_flop_count.py
+# recomputes them): column 0 of the seeded 1-degree workload (nAlts 100) and of
+# the 5-degree one (nAlts 50).  Columns differ by about 0.1% (branches).  A fixed
+# measure of the step's work: the kernel of this workload, which splits a level
+# over the species, solves the friction without pivoting, divides by short
+# reciprocals and repeats a few per-level terms in each of its groups.
 OPS_AUSM = {100: dict(add=351994, mul=540220, div=29130, sqrt=3232, trans=31057, cmp=137398),
             50: dict(add=178720, mul=273185, div=14880, sqrt=1632, trans=16157, cmp=68890)}
 # weights: +, -, *, min, max, compare 1; divide and sqrt 10; exp, log, pow,
@@ -219,13 +222,13 @@ def bench_ensemble(torch, solver, params, steps: int = 20, seed: int = 4) -> dic
     """The ragged ensemble: 64 members with nAlts drawn from 50..120 and 2592,
     10368 or 25920 columns each (gitm_amd.synth.ensemble), advanced as one
     batch.  Each member's columns tile the first min(n, 2592) columns of its
-    own seeded atmosphere.  The step's tile (workgroup size, short columns
-    per workgroup, where the RK4 carries live, persistent grid or not) is
-    autotuned on a probe batch; then a hipGraph holding ``steps`` x (batch
-    prep with per-member CFL steps + batch step) is replayed once and timed.
-    A batch step is one launch; the prep is two (the per-member step words
-    are reset, then the columns' CFL limits folded in).  Also timed: the same
-    steps at a fixed dt, one launch of ``steps`` steps."""
+    own seeded atmosphere.  A hipGraph holding ``steps`` x (batch prep with
+    per-member CFL steps + batch step) is replayed once and timed.  A batch
+    step is one launch per class of column heights, three here (columns of more
+    than 60 levels, of 60 and of 50 fit a CU in different numbers); the prep is
+    two (the per-member step words are reset, then the columns' CFL limits
+    folded in).  Also timed: the same steps at a fixed dt, ``steps`` steps per
+    launch."""
     from gitm_amd import synth, vertical
 
     mem = synth.ensemble(64, seed=seed)
@@ -240,7 +243,6 @@ def bench_ensemble(torch, solver, params, steps: int = 20, seed: int = 4) -> dic
     ncols = sum(int(d["temp"].shape[0]) for d in dev)
     levels = sum(int(d["temp"].shape[0]) * (int(d["temp"].shape[1]) - 4) for d in dev)
     b = vertical.VerticalBatch(solver, dev)
-    tune = b.autotune(params, "ausm")
     pp = synth.PrepParams()
     dt = torch.empty(len(dev), dtype=torch.float64, device="cuda")
     b.prepare(pp, dt_out=dt)
@@ -267,14 +269,11 @@ def bench_ensemble(torch, solver, params, steps: int = 20, seed: int = 4) -> dic
     fixed_ms = e0.elapsed_time(e1) / steps
     ok = all(bool(torch.isfinite(d["temp"]).all()) and bool((d["nds"] > 0).all())
              for d in dev)
-    tile = dict(zip(vertical.VerticalBatch.TILE_KEYS, b.tile()))
     del g
     b.close()
     return {"members": len(dev), "columns": ncols, "mean_n_alts": levels / ncols,
             "distinct_n_alts": sorted({int(d["temp"].shape[1]) - 4 for d in dev}),
-            "tile": tile,
-            "tiles_tried": {",".join(map(str, k)): round(v, 4) for k, v in tune.items()},
-            "launches_per_step": {"step": 1, "prep": 2},
+            "launches_per_step": {"step": 3, "prep": 2},
             "graph_steps": steps,
             "ms_per_step_graph_prep_and_step": graph_ms,
             "column_updates_per_s_graph": ncols / (graph_ms * 1e-3),
@@ -594,16 +593,18 @@ def bench_adjoint(torch, solver, steps: int = 10, seed: int = 5) -> dict:
 
 def roofline_fp64(spec, launch_ms: float) -> dict:
     """The FP64 roofline of the same launch: the weighted operation count of
-    the column code (OPS_AUSM) over the launch duration, against MI355X's
-    78.6 TFLOP/s FP64 vector peak.  This is the binding bound: the step's
-    intensity (about 56 weighted operations per algorithmic byte) is far
-    above the FP64 ridge (78.6e12 / 8e12 = 9.8 per byte)."""
+    the step with one lane per level (OPS_AUSM, a fixed measure of the work and
+    not the kernel's own instructions) over the launch duration, against
+    MI355X's 78.6 TFLOP/s FP64 vector peak.  Of the two rooflines it is the
+    nearer: the step's intensity (about 56 weighted operations per algorithmic
+    byte) is far above the FP64 ridge (78.6e12 / 8e12 = 9.8 per byte)."""
     ops = ops_per_column(spec.nalts) * spec.ncols
     raw = ops_per_column(spec.nalts, weighted=False) * spec.ncols
     achieved = ops / (launch_ms * 1e-3) / 1e12
     return {"bound": "fp64", "achieved": achieved, "peak": FP64_PEAK_TFLOPS,
             "unit": "TFLOP/s", "frac": achieved / FP64_PEAK_TFLOPS,
             "ops_per_launch": ops, "raw_ops_per_launch": raw,
+            "ops": "the step's work as counted with one lane per level",
             "weights": "+-*,min,max,cmp 1; div,sqrt 10; exp,log,pow,tanh 20",
             "intensity_ops_per_byte": ops / (bytes_per_column(spec.nalts) * spec.ncols),
             "binding": True}

@@ -340,8 +340,10 @@ extern "C" int gitm_vert_advance_host(gitm_vert_handle *h, const gitm_vert_param
 // hipGraph capture, serving loops).  Its scratch memory is the file-scope
 // array below, which every device the library runs on holds until the
 // process ends: the first 256 bytes hold the error word, the rest the RK4
-// carries that gitm_vert_advance keeps in its handle's scratch (ion carries
-// and the carries of columns taller than 188 levels).
+// carries that the kernels with one lane per level keep in device memory (ion
+// carries and the carries of columns taller than 188 levels).  The AUSM step
+// keeps its carries in registers but for ions above 226 levels; the limits are
+// the same for both solvers.
 // ---------------------------------------------------------------------------
 #include <mutex>
 

@@ -5,8 +5,8 @@
 
 namespace {
 
-// 768 threads hold the tallest column; three wavefronts per SIMD leave a lane
-// 168 registers.
+// 768 threads hold the tallest column; four wavefronts per SIMD leave a lane
+// 128 registers (76 B per lane spilled, 164 with ions).
 template <bool IONS>
 __global__ void __launch_bounds__(768, 4)
     vert_group_kernel(gv::KParams kp, gitm_vert_columns io) {

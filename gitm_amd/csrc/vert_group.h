@@ -13,8 +13,9 @@
 // keeps 530 registers live through the flux phase, so a SIMD holds one
 // wavefront, and a single wavefront leaves the FP64 pipe idle while it waits
 // for LDS, barriers and its register spills (47 % of its cycles issue a
-// vector instruction).  With two species a lane needs a third of that, a SIMD
-// holds three wavefronts and one's waits are another's work.
+// vector instruction).  With two species a lane makes do with 128, a SIMD's
+// registers hold four wavefronts and one's waits are another's work; at 100
+// levels LDS admits two columns per CU, three wavefronts per SIMD.
 //
 // The stage's state lives in LDS (a level's 17 fields side by side), so every
 // lane reads any level's field; what crosses levels or groups goes through

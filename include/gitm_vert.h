@@ -188,11 +188,11 @@ int gitm_vert_advance_host(gitm_vert_handle *h, const gitm_vert_params *p,
  * no library allocation.  It has no counterpart in the reference.  Its
  * scratch (the error word and the RK4 carries that gitm_vert_advance keeps in
  * its handle) is a fixed 64 MiB device array that every device the library
- * runs on holds until the process ends.  Runs that need more carries
- * return GITM_VERT_ESCRATCH before touching the device: with ion advection
- * more than 8,630 columns at nAlts = 50 or 4,481 at nAlts = 100; without,
- * only columns of nAlts > 188 need carries, at most 963 of them at nAlts =
- * 252.  Runs on the current device, asynchronously on
+ * runs on holds until the process ends.  Runs whose carries, with one lane
+ * per level, need more return GITM_VERT_ESCRATCH before touching the device
+ * (with either solver): with ion advection more than 8,630 columns at nAlts =
+ * 50 or 4,481 at nAlts = 100; without, only columns of nAlts > 188 count, at
+ * most 963 of them at nAlts = 252.  Runs on the current device, asynchronously on
  * `hip_stream` (NULL: the null stream); the kernels are those of
  * gitm_vert_advance, so results are identical.  Calls that overlap on one
  * device share the scratch and race: serialise them (one stream).

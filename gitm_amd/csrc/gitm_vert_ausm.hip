@@ -6,7 +6,7 @@
 namespace {
 
 // 768 threads hold the tallest column; four wavefronts per SIMD leave a lane
-// 128 registers (76 B per lane spilled, 164 with ions).
+// 128 registers (60 B per lane spilled, 164 with ions).
 template <bool IONS>
 __global__ void __launch_bounds__(768, 4)
     vert_group_kernel(gv::KParams kp, gitm_vert_columns io) {

@@ -319,8 +319,8 @@ GV_FN R limiter_mc(double beta, R up, R dn) {
 // device, whose comparisons it fails and whose minima it drops out of: as dn it
 // gives zero (q = 0), as up it leaves beta dn below zero and else zero (u =
 // -inf); a NaN thus changes no slope but its own cell's.
-// Eleven instructions, as many as a selection by the slopes' sign bits, which is
-// blind to NaN: the 1-degree horizontal step takes 4.24 ms in place of 4.19, the
+// Ten instructions, about as many as a selection by the slopes' sign bits, which
+// is blind to NaN: the 1-degree horizontal step takes 4.24 ms in place of 4.19, the
 // 1-degree AUSM step the same; comparisons of the slopes, which become branches,
 // cost 6 and 4 %.
 GV_FN double limiter_flat(double beta, double up, double dn) {
